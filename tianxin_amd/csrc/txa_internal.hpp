@@ -67,6 +67,13 @@ struct MeshBlock {
   int64_t nelem = 0, elem_begin = 0, conn_begin = 0;
 };
 
+// Launch shape of the lattice kernels on a brick (txa_q1_hex8.hip): tile shape and vertex layers per
+// z slab of the row-owner kernel, and the slab height of the residual kernel; 0: no lattice kernel.
+struct Q1Plan {
+  bool small = false;
+  int zc = 0, zc_f = 0;
+};
+
 // A mesh with its DOF map and CRS graph, resident on the device: a structured brick,
 // or uploaded connectivity of one or several element blocks.
 struct Mesh {
@@ -98,6 +105,7 @@ struct Mesh {
   DevBuf<int32_t> col;
   int perm_width = 0;         // bytes per row of the stencil slot map (27*nfields rounded up to 16)
   DevBuf<uint8_t> perm;       // [ndofs][perm_width] position of each stencil neighbour in the row, 255 = absent
+  Q1Plan q1;                  // one-field HEX8 / TET4 bricks
   int nperm_w = 0;            // entries per node of nperm
   DevBuf<uint16_t> nperm;     // 3-field HEX8 / HEX27: [nodes][nperm_w] position of (neighbour, field 0) in the node's rows
   DevBuf<double> cell_geom;   // 3-field HEX8 bricks of parallelepiped cells: [cells][10] scaled cofactors, |det J|
@@ -236,6 +244,7 @@ bool elastic_supported(const Mesh &m, const txa_assembly_args &a);
 size_t elastic_workspace_bytes(const Mesh &m, int precision, bool want_f, bool want_vals);
 void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws);
 // Q1 diffusion fast path and batches (txa_q1_hex8.hip)
+Q1Plan q1_plan(const Mesh &m, int ncu);
 void launch_q1_hex8_diffusion(Mesh &m, const txa_assembly_args &a, hipStream_t s);
 // uploaded one-field HEX8 / TET4 diffusion by node patches (txa_patch.hip)
 void patch_build(Mesh &m, hipStream_t s);

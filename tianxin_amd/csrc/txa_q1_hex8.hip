@@ -18,27 +18,28 @@
 
 #include <algorithm>
 #include <cstring>
+#include <functional>
+#include <queue>
 
 namespace txa {
 namespace {
 
 // Element tiles: TX vertex columns along x by TY along y, one element lane and one owner
-// lane per column.  Single meshes take 32 x 8 (a 16 x 16 tile recomputes fewer halo
-// elements but ran 1.5% slower at 256^3); batches take 32 x 8 or 16 x 16, whichever the
-// autotuner times faster (16 x 16 covers meshes 16-64 cells wide with fewer idle lanes).
-constexpr int NE = 256;                        // element lanes = owner lanes
-constexpr int NT = 2 * NE;                     // block: 4 element waves + 4 owner waves
-constexpr int kTX = 32;                        // tile width of the single-mesh kernels
-template <int TXV>
+// lane per column (NE = TX TY of each), TX - 1 by TY - 1 columns owned.
+template <int TXV, int NEV>
 struct Tile {
-  static_assert(TXV == 16 || TXV == 32, "tile width");
-  static constexpr int TX = TXV, TY = NE / TXV;
+  static_assert((TXV == 16 || TXV == 32) && (NEV == 128 || NEV == 256), "tile shape");
+  static constexpr int NE = NEV, NT = 2 * NEV;   // element lanes = owner lanes; block: both roles
+  static constexpr int TX = TXV, TY = NEV / TXV;
   // owner groups (the TX lanes of one x line of owners, TX-1 of them own rows): doubles per
   // group's row buffer, TX-1 rows of at most 27 entries, then a spare slot for the entries a
   // row does not have
   static constexpr int ROWBUF = 27 * TX, ROWBUF_SPARE = 27 * (TX - 1);
   static constexpr int NOWN = TX * (TY - 1);   // owner lanes with rows
 };
+using Wide = Tile<32, 256>;     // one workgroup per CU (LDS)
+using Square = Tile<16, 256>;   // one workgroup per CU, batches
+using Small = Tile<16, 128>;    // two workgroups per CU
 using namespace q1elem;
 // element kinds of the lattice kernels: TXA_HEX8 (general trilinear cells), TXA_TET4 (six
 // tets per cell) and hex8 cells that are all parallelepipeds (constant metric per cell)
@@ -50,7 +51,7 @@ constexpr int NSTAGE = 44;   // per element: 36 packed K, then 8 FP64 R (FP64) o
 template <typename Real>
 constexpr int stage_slots() { return sizeof(Real) == 4 ? 2 : 1; }
 
-constexpr int kTargetBlocks = 2560;   // z slabs are sized to give about this many workgroups
+constexpr int kTargetBlocks = 2560;   // large meshes: z slabs are sized to give about this many workgroups
 
 struct Q1DiffParams {
   int nx, ny, nz;
@@ -75,6 +76,14 @@ __device__ __forceinline__ constexpr int tet_v(int t, int j) {
   return T[t][j];
 }
 
+// a b - c d and a0 b0 + a1 b1 + a2 b2 with their fused operations written out: left to the
+// compiler, which product is fused depends on what else the kernel around it uses, and the
+// residual-only kernel has to give the row-owner kernel's f bit for bit.
+__device__ __forceinline__ double diff2(double a, double b, double c, double d) { return __builtin_fma(a, b, -(c * d)); }
+__device__ __forceinline__ double dot3(double a0, double b0, double a1, double b1, double a2, double b2) {
+  return __builtin_fma(a2, b2, __builtin_fma(a1, b1, a0 * b0));
+}
+
 // The six linear tets of one cell, assembled into the cell's 8x8 matrix (pairs
 // not joined by a tet edge stay zero).  Constant gradients: grad N_j = cof[:,j]/det
 // (j = 1..3), grad N_0 = -(sum); measure w |det| with w = 1/6; the degree-2
@@ -84,10 +93,9 @@ template <typename Real, bool TRANS, bool UNIT, class Mid>
 __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double (&u)[8], const double (&ud)[8],
                                           const double (&k)[6], double rhoc, double src, double alpha, double beta,
                                           Hex8Out<Real, TRANS> &o, Mid &&mid) {
-  constexpr bool kFlux = flux_residual<Real>();
   mid();
   Real K[36], M[TRANS ? 36 : 1];
-  double F[8], Rf[8];   // source load; FP64 residual K u + M udot of the FP32 form
+  double F[8], Rf[8];   // source load; residual K u + M udot, from the flux
 #pragma unroll
   for (int i = 0; i < 36; ++i) { K[i] = Real(0); if (TRANS) M[i] = Real(0); }
 #pragma unroll
@@ -100,32 +108,32 @@ __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double 
 #pragma unroll
       for (int j = 0; j < 3; ++j) J[d][j] = X[d][tet_v(t, j + 1)] - X[d][tet_v(t, 0)];
     double c[3][3];
-    c[0][0] = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-    c[0][1] = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-    c[0][2] = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-    c[1][0] = J[0][2] * J[2][1] - J[0][1] * J[2][2];
-    c[1][1] = J[0][0] * J[2][2] - J[0][2] * J[2][0];
-    c[1][2] = J[0][1] * J[2][0] - J[0][0] * J[2][1];
-    c[2][0] = J[0][1] * J[1][2] - J[0][2] * J[1][1];
-    c[2][1] = J[0][2] * J[1][0] - J[0][0] * J[1][2];
-    c[2][2] = J[0][0] * J[1][1] - J[0][1] * J[1][0];
-    const double det = J[0][0] * c[0][0] + J[0][1] * c[0][1] + J[0][2] * c[0][2];
+    c[0][0] = diff2(J[1][1], J[2][2], J[1][2], J[2][1]);
+    c[0][1] = diff2(J[1][2], J[2][0], J[1][0], J[2][2]);
+    c[0][2] = diff2(J[1][0], J[2][1], J[1][1], J[2][0]);
+    c[1][0] = diff2(J[0][2], J[2][1], J[0][1], J[2][2]);
+    c[1][1] = diff2(J[0][0], J[2][2], J[0][2], J[2][0]);
+    c[1][2] = diff2(J[0][1], J[2][0], J[0][0], J[2][1]);
+    c[2][0] = diff2(J[0][1], J[1][2], J[0][2], J[1][1]);
+    c[2][1] = diff2(J[0][2], J[1][0], J[0][0], J[1][2]);
+    c[2][2] = diff2(J[0][0], J[1][1], J[0][1], J[1][0]);
+    const double det = dot3(J[0][0], c[0][0], J[0][1], c[0][1], J[0][2], c[0][2]);
     const double sg = det < 0.0 ? -1.0 : 1.0;
     const double vol = det * sg / 6.0;                 // sum of the weighted measure
     const double cw64 = k[t] * sg * recip(det) / 6.0;
     const Real cw = Real(cw64);
-    if constexpr (kFlux) {
+    {
       // FP64: grad u (times det) = cof (u_j - u_0), R_j = cw g_j . (cof du), R_0 = -(R_1 + R_2 + R_3);
       // mass rho_c |T| / 20 (udot_a + sum_b udot_b)
       const double du0 = u[tet_v(t, 1)] - u[tet_v(t, 0)], du1 = u[tet_v(t, 2)] - u[tet_v(t, 0)],
                    du2 = u[tet_v(t, 3)] - u[tet_v(t, 0)];
       double tt[3];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) tt[i] = cw64 * (c[i][0] * du0 + c[i][1] * du1 + c[i][2] * du2);
+      for (int i = 0; i < 3; ++i) tt[i] = cw64 * dot3(c[i][0], du0, c[i][1], du1, c[i][2], du2);
       double rs = 0.0;
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const double r = c[0][j] * tt[0] + c[1][j] * tt[1] + c[2][j] * tt[2];
+        const double r = dot3(c[0][j], tt[0], c[1][j], tt[1], c[2][j], tt[2]);
         Rf[tet_v(t, j + 1)] += r;
         rs += r;
       }
@@ -134,7 +142,7 @@ __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double 
         const double sud = ud[tet_v(t, 0)] + ud[tet_v(t, 1)] + ud[tet_v(t, 2)] + ud[tet_v(t, 3)];
         const double mw = rhoc * vol * 0.05;
 #pragma unroll
-        for (int a = 0; a < 4; ++a) Rf[tet_v(t, a)] += mw * (sud + ud[tet_v(t, a)]);
+        for (int a = 0; a < 4; ++a) Rf[tet_v(t, a)] = __builtin_fma(mw, sud + ud[tet_v(t, a)], Rf[tet_v(t, a)]);
       }
     }
     Real g[4][3];
@@ -154,21 +162,8 @@ __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double 
       }
     }
   }
-  if constexpr (kFlux) {
 #pragma unroll
-    for (int a = 0; a < 8; ++a) o.R[a] = Rf[a] - F[a];
-  } else {
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      Real r = Real(0);
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        r += K[sym8(a, b)] * Real(u[b]);
-        if (TRANS) r += M[sym8(a, b)] * Real(ud[b]);
-      }
-      o.R[a] = double(r) - F[a];
-    }
-  }
+  for (int a = 0; a < 8; ++a) o.R[a] = Rf[a] - F[a];
 #pragma unroll
   for (int i = 0; i < 36; ++i)
     o.K[i] = TRANS ? Real(beta) * K[i] + Real(alpha) * M[i] : (UNIT ? K[i] : Real(beta) * K[i]);
@@ -246,11 +241,11 @@ __device__ __forceinline__ RowMeta load_meta(const Q1DiffParams &p, int32_t L) {
 // The range is stored in chunks of TX entries aligned to TX entries.  It removes the partial lines
 // inside a range (WRITE_SIZE 4.32 -> 3.81 GB at 256^3, the bytes of f and the values):
 // about 1% faster in both the FP32 and the FP64 kernels at 256^3.
-template <int TXV>
+template <class T>
 __device__ __forceinline__ void emit_rows(const Q1DiffParams &p, const RowMeta &m, const double (&acc)[27], double r,
                                           double *rowbuf, int grp) {
-  constexpr int GW = TXV;   // lanes per group
-  constexpr int ROWBUF = Tile<TXV>::ROWBUF, ROWBUF_SPARE = Tile<TXV>::ROWBUF_SPARE;
+  constexpr int GW = T::TX;   // lanes per group
+  constexpr int ROWBUF = T::ROWBUF, ROWBUF_SPARE = T::ROWBUF_SPARE;
   constexpr uint64_t GMASK = (1ull << GW) - 1;
   const int lane = threadIdx.x & 63, gl = lane & (GW - 1), gi = lane / GW;
   const bool act = m.L >= 0;
@@ -343,12 +338,12 @@ __device__ __forceinline__ RowMeta load_meta_flat(const Q1DiffParams &p, int32_t
 // position, [3..9] the slot map words 0-6 with the row length in the top byte of
 // word 6 (byte 27 of the map, which carries no slot).
 constexpr int MWORDS = 10;
-template <int TXV>
-constexpr int mslot() { return MWORDS * Tile<TXV>::NOWN; }
+template <class T>
+constexpr int mslot() { return MWORDS * T::NOWN; }
 
-template <int TXV>
+template <class T>
 __device__ __forceinline__ void put_meta(uint32_t *ms, int t, const RowMeta &m) {
-  constexpr int NOWN = Tile<TXV>::NOWN;
+  constexpr int NOWN = T::NOWN;
   ms[t] = static_cast<uint32_t>(m.L);
   ms[NOWN + t] = static_cast<uint32_t>(static_cast<uint64_t>(m.base));
   ms[2 * NOWN + t] = static_cast<uint32_t>(static_cast<uint64_t>(m.base) >> 32);
@@ -357,9 +352,9 @@ __device__ __forceinline__ void put_meta(uint32_t *ms, int t, const RowMeta &m) 
   ms[9 * NOWN + t] = (m.w[6] & 0x00ffffffu) | (static_cast<uint32_t>(m.end - m.base) << 24);
 }
 
-template <int TXV>
+template <class T>
 __device__ __forceinline__ RowMeta get_meta(const uint32_t *ms, int t) {
-  constexpr int NOWN = Tile<TXV>::NOWN;
+  constexpr int NOWN = T::NOWN;
   RowMeta m;
   m.L = static_cast<int32_t>(ms[t]);
   m.base = static_cast<int64_t>(ms[NOWN + t] | static_cast<uint64_t>(ms[2 * NOWN + t]) << 32);
@@ -381,10 +376,10 @@ __device__ __forceinline__ constexpr bool first_touch(int CX, int CY, int x, int
 // in the order (1,1), (0,1), (1,0), (0,0): the first contribution to a slot of the
 // next layer's row (accn, rn) or to the upper stencil layer of this row (acc[18..26])
 // is stored rather than added, so those slots need no clearing between layers.
-template <int CX, int CY, typename Real>
+template <class T, int CX, int CY, typename Real>
 __device__ __forceinline__ void take_corner(const Real *s, int col, double (&acc)[27], double (&accn)[18], double &rc,
                                             double &rn) {
-  constexpr int alo = CX + 2 * CY, ahi = alo + 4;
+  constexpr int NE = T::NE, alo = CX + 2 * CY, ahi = alo + 4;
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
     const int bx = b & 1, by = (b >> 1) & 1, bz = (b >> 2) & 1;
@@ -407,9 +402,9 @@ __device__ __forceinline__ void take_corner(const Real *s, int col, double (&acc
 // Residual of the FP32 form: the stage holds, per element column c, the x-pair sums
 // P_c[by + 2 bz] = R_c[1 + 2by + 4bz] + R_{c+1}[2by + 4bz] (FP64) of the element and its
 // +x neighbour, so the owner at corner (1,1) of column c adds two values per vertex layer.
-template <int TXV, typename Real>
+template <class T, typename Real>
 __device__ __forceinline__ void take_pairs(const Real *s, int col, double &rc, double &rn) {
-  constexpr int TX = TXV;
+  constexpr int TX = T::TX, NE = T::NE;
   if constexpr (flux_residual<Real>()) {
     const double *ps = reinterpret_cast<const double *>(s + 36 * NE);
     rc += ps[1 * NE + col] + ps[0 * NE + col + TX];
@@ -452,10 +447,10 @@ __device__ __forceinline__ void load_face_lids(const Q1DiffParams &p, int64_t n0
 // owner wave to one layer of stores in flight.  The element waves therefore load
 // the owners' LIDs, row pointers and slot maps and publish them with the layer.
 // UNIT: the steady tangent with beta = 1 (the element matrix is stored unscaled).
-template <int TXV, int KIND, typename Real, bool TRANS, bool UNIT>
+template <class T, int KIND, typename Real, bool TRANS, bool UNIT>
 __device__ __forceinline__ void spec_block(const Q1DiffParams &p, int bx, int by, int bz, Real *stage,
                                            double *rowbuf, uint32_t *meta) {
-  constexpr int TX = Tile<TXV>::TX, TY = Tile<TXV>::TY, NOWN = Tile<TXV>::NOWN, MSLOT = mslot<TXV>();
+  constexpr int TX = T::TX, TY = T::TY, NE = T::NE, NOWN = T::NOWN, MSLOT = mslot<T>();
   constexpr int NSLOT = stage_slots<Real>();
   const bool is_elem = threadIdx.x < NE;
   const int t = is_elem ? threadIdx.x : threadIdx.x - NE;
@@ -574,7 +569,7 @@ __device__ __forceinline__ void spec_block(const Q1DiffParams &p, int bx, int by
         for (int i = 0; i < (flux_residual<Real>() ? 4 : 8); ++i)
           reinterpret_cast<double *>(st + 36 * NE)[i * NE + t] = o.R[i];
       }
-      if (t < NOWN) put_meta<TXV>(meta + sl * MSLOT, t, om);
+      if (t < NOWN) put_meta<T>(meta + sl * MSLOT, t, om);
       Lo = Lo_next;
       __syncthreads();   // layer ez is in the stage (two slots: the owners are also done with layer ez-1)
     }
@@ -597,14 +592,14 @@ __device__ __forceinline__ void spec_block(const Q1DiffParams &p, int bx, int by
         const Real *st = stage + sl * (NSTAGE * NE);
         RowMeta m;
         if (owner) {
-          m = get_meta<TXV>(meta + sl * MSLOT, t);
-          take_corner<1, 1>(st, t, acc, accn, rc, rn);
-          take_corner<0, 1>(st, t + 1, acc, accn, rc, rn);
-          take_corner<1, 0>(st, t + TX, acc, accn, rc, rn);
-          take_corner<0, 0>(st, t + TX + 1, acc, accn, rc, rn);
-          take_pairs<TXV>(st, t, rc, rn);
+          m = get_meta<T>(meta + sl * MSLOT, t);
+          take_corner<T, 1, 1>(st, t, acc, accn, rc, rn);
+          take_corner<T, 0, 1>(st, t + 1, acc, accn, rc, rn);
+          take_corner<T, 1, 0>(st, t + TX, acc, accn, rc, rn);
+          take_corner<T, 0, 0>(st, t + TX + 1, acc, accn, rc, rn);
+          take_pairs<T>(st, t, rc, rn);
         }
-        if (e >= k0) emit_rows<TXV>(p, m, acc, rc, rowbuf, t / TX);
+        if (e >= k0) emit_rows<T>(p, m, acc, rc, rowbuf, t / TX);
 #pragma unroll
         for (int s = 0; s < 18; ++s) acc[s] = accn[s];
         rc = rn;
@@ -615,20 +610,116 @@ __device__ __forceinline__ void spec_block(const Q1DiffParams &p, int bx, int by
     // the top vertex layer of the mesh has no element layer above it
     if (k1 == p.nz + 1) {
       RowMeta m;
-      if (owner) m = get_meta<TXV>(meta + (NSLOT == 2 ? ((ez1 + 1) & 1) : 0) * MSLOT, t);
-      emit_rows<TXV>(p, m, acc, rc, rowbuf, t / TX);
+      if (owner) m = get_meta<T>(meta + (NSLOT == 2 ? ((ez1 + 1) & 1) : 0) * MSLOT, t);
+      emit_rows<T>(p, m, acc, rc, rowbuf, t / TX);
     }
   }
 }
 
 
-template <int KIND, typename Real, bool TRANS, bool UNIT>
-__global__ __launch_bounds__(NT) void k_q1_hex8_diffusion(Q1DiffParams p) {
-  using T = Tile<kTX>;
-  __shared__ __align__(16) Real stage[stage_slots<Real>() * NSTAGE * NE];
+// Tile of a workgroup.  Consecutive workgroups go to the eight XCDs in turn, and with x fastest and
+// a multiple of four tiles along x, the tiles of one XCD are few x stripes of the mesh: the same
+// work then takes up to 1.7 times as long (FP64 240^3, eight wide tiles along x: 1960 us against
+// 1212 us y fastest; 112^3, four: 226 against 165).  Wide tiles go y fastest where there are four
+// or more along x (256^3, nine: 1388 -> 1343 us; 200^3 752 -> 726), small ones x fastest (2% faster
+// than y fastest) with each line of tiles rotated by one where x is a multiple of four (112^3 209
+// -> 138 us).
+constexpr int kYFastest = 4;
+template <class T>
+__device__ __forceinline__ int3 tile_of_block() {
+  const int gx = gridDim.x, gy = gridDim.y;
+  const int l = blockIdx.x + gx * blockIdx.y, bz = blockIdx.z;
+  if (T::TX == 32 && gx >= kYFastest) return make_int3(l / gy, l % gy, bz);
+  const int y = l / gx, x = l % gx;
+  return make_int3(T::TX == 16 && gx % 4 == 0 ? (x + y) % gx : x, y, bz);
+}
+
+template <class T, int KIND, typename Real, bool TRANS, bool UNIT>
+__global__ __launch_bounds__(T::NT, 2) void k_q1_hex8_diffusion(Q1DiffParams p) {
+  __shared__ __align__(16) Real stage[stage_slots<Real>() * NSTAGE * T::NE];
   __shared__ double rowbuf[(T::TY - 1) * T::ROWBUF];
-  __shared__ uint32_t meta[stage_slots<Real>() * mslot<kTX>()];
-  spec_block<kTX, KIND, Real, TRANS, UNIT>(p, blockIdx.x, blockIdx.y, blockIdx.z, stage, rowbuf, meta);
+  __shared__ uint32_t meta[stage_slots<Real>() * mslot<T>()];
+  const int3 b = tile_of_block<T>();
+  spec_block<T, KIND, Real, TRANS, UNIT>(p, b.x, b.y, b.z, stage, rowbuf, meta);
+}
+
+// Residual alone (vals null): the same element routine on the same tiles, without the matrix
+// stage, the row buffers and the slot maps.  One role: every thread computes an element column,
+// puts its eight residual entries in LDS (two slots: one barrier per layer) and, if it owns the
+// tile's vertex column (tx + 1, ty + 1), adds the four columns' entries in the order of the
+// row-owner kernel, so f is the same bit for bit.  Bound by the element arithmetic: 32 KB of LDS
+// instead of 147 KB leaves two or more workgroups per CU by registers where the row-owner kernel
+// had one with half its waves idle. 
+template <int KIND, typename Real, bool TRANS>
+__global__ __launch_bounds__(Wide::NE, 2) void k_q1_residual(Q1DiffParams p) {
+  constexpr int TX = Wide::TX, TY = Wide::TY, NE = Wide::NE;
+  __shared__ double rs[2][8][NE];
+  const int t = threadIdx.x, tx = t % TX, ty = t / TX;
+  const int3 blk = tile_of_block<Wide>();
+  const int ex = -1 + blk.x * (TX - 1) + tx, ey = -1 + blk.y * (TY - 1) + ty;
+  const int64_t sx = p.nx + 1, sxy = sx * (p.ny + 1);
+  const int k0 = blk.z * p.zc, k1 = min(k0 + p.zc, p.nz + 1);
+  const int ez0 = max(k0 - 1, 0), ez1 = min(k1 - 1, p.nz - 1);
+  const bool evalid = ex >= 0 && ex < p.nx && ey >= 0 && ey < p.ny;
+  const int64_t col0 = evalid ? ex + sx * ey : 0;
+  const int64_t cell0 = evalid ? ex + static_cast<int64_t>(p.nx) * ey : 0;
+  const int64_t sz = static_cast<int64_t>(p.nx) * p.ny;
+  const int oi = ex + 1, oj = ey + 1;
+  const bool owns = tx < TX - 1 && ty < TY - 1 && oi <= p.nx && oj <= p.ny;
+  const int64_t ocol = owns ? oi + sx * oj : 0;
+  Face<TRANS> fb, ft;
+  int32_t L[4];
+  load_face_lids(p, col0 + sxy * ez0, sx, L);
+  load_face(p, col0 + sxy * ez0, sx, L, fb);
+  load_face_lids(p, col0 + sxy * (ez0 + 1), sx, L);   // LIDs run one layer ahead of the faces
+  double rc = 0.0, rn = 0.0;
+  for (int ez = ez0; ez <= ez1; ++ez) {
+    load_face(p, col0 + sxy * (ez + 1), sx, L, ft);
+    load_face_lids(p, col0 + sxy * min(ez + 2, p.nz), sx, L);
+    CellCoef<KIND> kc;
+    load_coef<KIND>(p, cell0 + sz * ez, kc);
+    const int32_t Lo = p.lid[ocol + sxy * ez];
+    double(&st)[8][NE] = rs[ez & 1];
+    if (evalid) {
+      double X[3][8], u[8], ud[8];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) { X[d][v] = fb.x[d][v]; X[d][v + 4] = ft.x[d][v]; }
+        u[v] = fb.u[v]; u[v + 4] = ft.u[v];
+        ud[v] = fb.ud[v]; ud[v + 4] = ft.ud[v];
+      }
+      Hex8Out<Real, TRANS> o;
+      cell_element<KIND, Real, TRANS, true>(p, kc, X, u, ud, o, [] {});
+#pragma unroll
+      for (int a = 0; a < 8; ++a) st[a][t] = o.R[a];
+    } else {
+#pragma unroll
+      for (int a = 0; a < 8; ++a) st[a][t] = 0.0;
+    }
+    fb = ft;
+    __syncthreads();   // layer ez is in its slot; the slot of layer ez - 1 is free after the next one
+    if (owns) {
+      // corners in the row-owner kernel's order (1,1), (0,1), (1,0), (0,0)
+      if constexpr (flux_residual<Real>()) {
+        rc += (st[3][t] + st[2][t + 1]) + (st[1][t + TX] + st[0][t + TX + 1]);
+        rn = (st[7][t] + st[6][t + 1]) + (st[5][t + TX] + st[4][t + TX + 1]);
+      } else {
+        rc += st[3][t];
+        rc += st[2][t + 1];
+        rc += st[1][t + TX];
+        rc += st[0][t + TX + 1];
+        rn = st[7][t];
+        rn += st[6][t + 1];
+        rn += st[5][t + TX];
+        rn += st[4][t + TX + 1];
+      }
+      if (ez >= k0) p.f[Lo] = rc;
+    }
+    rc = rn;
+  }
+  // the top vertex layer of the mesh has no element layer above it
+  if (owns && k1 == p.nz + 1) p.f[p.lid[ocol + sxy * p.nz]] = rc;
 }
 
 // ============================================================================
@@ -664,13 +755,12 @@ __device__ __forceinline__ void leave_queue(BatchQueue *q) {
 // One element kind per launch (FP64, transient or general-cell batches, and batches of one
 // kind): a kernel holding both bodies spills there.  FP32 steady batches of both kinds with
 // parallelepiped hex8 cells take k_q1_batch_mixed.
-template <int TXV, int KIND, typename Real, bool TRANS>
-__global__ __launch_bounds__(NT) void k_q1_batch_spec(const Q1DiffParams *__restrict__ prm,
+template <class T, int KIND, typename Real, bool TRANS>
+__global__ __launch_bounds__(T::NT, 2) void k_q1_batch_spec(const Q1DiffParams *__restrict__ prm,
                                                       const int4 *__restrict__ items, int nitems, BatchQueue *q) {
-  using T = Tile<TXV>;
-  __shared__ __align__(16) Real stage[stage_slots<Real>() * NSTAGE * NE];
+  __shared__ __align__(16) Real stage[stage_slots<Real>() * NSTAGE * T::NE];
   __shared__ double rowbuf[(T::TY - 1) * T::ROWBUF];
-  __shared__ uint32_t meta[stage_slots<Real>() * mslot<TXV>()];
+  __shared__ uint32_t meta[stage_slots<Real>() * mslot<T>()];
   __shared__ int slot;
   for (;;) {
     const int it = fetch_item(q, &slot);
@@ -678,7 +768,7 @@ __global__ __launch_bounds__(NT) void k_q1_batch_spec(const Q1DiffParams *__rest
     const int4 w = items[it];
     const Q1DiffParams &p = prm[w.x];
     if (w.w * p.zc > p.nz) continue;   // slab past the mesh: nothing to do (uniform over the block)
-    spec_block<TXV, KIND, Real, TRANS, false>(p, w.y, w.z, w.w, stage, rowbuf, meta);
+    spec_block<T, KIND, Real, TRANS, false>(p, w.y, w.z, w.w, stage, rowbuf, meta);
     __syncthreads();
   }
   leave_queue(q);
@@ -688,13 +778,12 @@ __global__ __launch_bounds__(NT) void k_q1_batch_spec(const Q1DiffParams *__rest
 // meshes, tile x, tile y, slab) items over hex8 and tet4 meshes, longest first.
 constexpr int kMixedTet = 1 << 30;
 
-template <int TXV, int HEXKIND, typename Real, bool TRANS>
-__global__ __launch_bounds__(NT) void k_q1_batch_mixed(const Q1DiffParams *__restrict__ prm,
+template <class T, int HEXKIND, typename Real, bool TRANS>
+__global__ __launch_bounds__(T::NT, 2) void k_q1_batch_mixed(const Q1DiffParams *__restrict__ prm,
                                                        const int4 *__restrict__ items, int nitems, BatchQueue *q) {
-  using T = Tile<TXV>;
-  __shared__ __align__(16) Real stage[stage_slots<Real>() * NSTAGE * NE];
+  __shared__ __align__(16) Real stage[stage_slots<Real>() * NSTAGE * T::NE];
   __shared__ double rowbuf[(T::TY - 1) * T::ROWBUF];
-  __shared__ uint32_t meta[stage_slots<Real>() * mslot<TXV>()];
+  __shared__ uint32_t meta[stage_slots<Real>() * mslot<T>()];
   __shared__ int slot;
   for (;;) {
     const int it = fetch_item(q, &slot);
@@ -703,8 +792,8 @@ __global__ __launch_bounds__(NT) void k_q1_batch_mixed(const Q1DiffParams *__res
     const bool tet = (w.x & kMixedTet) != 0;
     const Q1DiffParams &p = prm[w.x & (kMixedTet - 1)];
     if (w.w * p.zc > p.nz) continue;   // slab past the mesh: nothing to do (uniform over the block)
-    if (tet) spec_block<TXV, TXA_TET4, Real, TRANS, false>(p, w.y, w.z, w.w, stage, rowbuf, meta);
-    else spec_block<TXV, HEXKIND, Real, TRANS, false>(p, w.y, w.z, w.w, stage, rowbuf, meta);
+    if (tet) spec_block<T, TXA_TET4, Real, TRANS, false>(p, w.y, w.z, w.w, stage, rowbuf, meta);
+    else spec_block<T, HEXKIND, Real, TRANS, false>(p, w.y, w.z, w.w, stage, rowbuf, meta);
     __syncthreads();
   }
   leave_queue(q);
@@ -762,18 +851,29 @@ __global__ void k_cell_affine(int nx, int ny, int nz, int64_t nv, const double *
 }
 
 // Element and owner waves split in both precisions (the stage is double-buffered in FP32).
-template <int KIND>
+template <class T, int KIND>
 void launch_kind(const Q1DiffParams &p, dim3 grid, int precision, bool trans, hipStream_t s) {
   const bool unit = p.beta == 1.0;
   if (precision == TXA_FP64) {
-    if (trans) hipLaunchKernelGGL((k_q1_hex8_diffusion<KIND, double, true, false>), grid, dim3(NT), 0, s, p);
-    else if (unit) hipLaunchKernelGGL((k_q1_hex8_diffusion<KIND, double, false, true>), grid, dim3(NT), 0, s, p);
-    else hipLaunchKernelGGL((k_q1_hex8_diffusion<KIND, double, false, false>), grid, dim3(NT), 0, s, p);
+    if (trans) hipLaunchKernelGGL((k_q1_hex8_diffusion<T, KIND, double, true, false>), grid, dim3(T::NT), 0, s, p);
+    else if (unit) hipLaunchKernelGGL((k_q1_hex8_diffusion<T, KIND, double, false, true>), grid, dim3(T::NT), 0, s, p);
+    else hipLaunchKernelGGL((k_q1_hex8_diffusion<T, KIND, double, false, false>), grid, dim3(T::NT), 0, s, p);
   } else {
     // FP32 scales by beta in every case: without the 36 multiplies the compiler's schedule
     // of the unit-beta instance spills (47 registers) where the scaled one fits in 240
-    if (trans) hipLaunchKernelGGL((k_q1_hex8_diffusion<KIND, float, true, false>), grid, dim3(NT), 0, s, p);
-    else hipLaunchKernelGGL((k_q1_hex8_diffusion<KIND, float, false, false>), grid, dim3(NT), 0, s, p);
+    if (trans) hipLaunchKernelGGL((k_q1_hex8_diffusion<T, KIND, float, true, false>), grid, dim3(T::NT), 0, s, p);
+    else hipLaunchKernelGGL((k_q1_hex8_diffusion<T, KIND, float, false, false>), grid, dim3(T::NT), 0, s, p);
+  }
+}
+
+template <int KIND>
+void launch_residual(const Q1DiffParams &p, dim3 grid, int precision, bool trans, hipStream_t s) {
+  if (precision == TXA_FP64) {
+    if (trans) hipLaunchKernelGGL((k_q1_residual<KIND, double, true>), grid, dim3(Wide::NE), 0, s, p);
+    else hipLaunchKernelGGL((k_q1_residual<KIND, double, false>), grid, dim3(Wide::NE), 0, s, p);
+  } else {
+    if (trans) hipLaunchKernelGGL((k_q1_residual<KIND, float, true>), grid, dim3(Wide::NE), 0, s, p);
+    else hipLaunchKernelGGL((k_q1_residual<KIND, float, false>), grid, dim3(Wide::NE), 0, s, p);
   }
 }
 
@@ -794,12 +894,9 @@ Q1DiffParams make_params(const Mesh &m, const txa_assembly_args &a, int zc) {
   return p;
 }
 
-// tiles of width tx (height 256 / tx) over a brick's vertex columns
-inline int tiles_x(const Mesh &m, int tx = kTX) { return (m.nx + 1 + tx - 2) / (tx - 1); }
-inline int tiles_y(const Mesh &m, int tx = kTX) {
-  const int ty = NE / tx;
-  return (m.ny + 1 + ty - 2) / (ty - 1);
-}
+// tiles of tx x ty columns (one fewer owned each way) over a brick's vertex columns
+inline int tiles_x(const Mesh &m, int tx) { return (m.nx + 1 + tx - 2) / (tx - 1); }
+inline int tiles_y(const Mesh &m, int ty) { return (m.ny + 1 + ty - 2) / (ty - 1); }
 
 }  // namespace
 
@@ -819,20 +916,109 @@ bool brick_cells_affine(const Mesh &m, hipStream_t s) {
   return h != 0;
 }
 
+// Tile shape and vertex layers per z slab of the single-mesh kernels, decided once per mesh with
+// its graph.  Costs are in layer steps of a wide tile (about 4 us, 6.5 us for general cells).
+//
+// Wide tiles, one workgroup per CU (LDS).  Large meshes (slabs of 8 or more layers give over four
+// workgroups per slot): slabs for about kTargetBlocks workgroups; taller slabs recompute less and
+// the launch's tail is short against the whole.  Smaller meshes leave CUs idle or end in a nearly
+// empty second round that way (32^3: 50 workgroups, 9 steps in a row), so the slab height is the
+// one whose workgroups, handed in order to the first free slot, end first; a tile counts half its
+// cost for its first vertex column and the rest by the columns it owns.
+//
+// Small tiles, two workgroups per CU: they share the CU, so the whole counts as throughput, half a
+// slab as tail, and a slab ends no sooner than its own steps; with at most one per CU the steps
+// are shorter.  Parallelepiped cells (bound by the layer's latency and the stores)
+// run 4-40% faster on them at every size (two workgroups' phases interleave, FP32 64^3 59 -> 45 us,
+// 128^3 237 -> 194, 256^3 1319 -> 1290), general cells and tets (bound by the element arithmetic;
+// a small tile recomputes 3% more) only where the wide tiles fit the mesh badly.
+//
+// Start (wide, x fastest, fixed 8-layer slabs) -> this plan: steady FP64 cubes 16^3 29.5 -> 20 us,
+// 32^3 45 -> 20, 64^3 59 -> 46, 97^3 177 -> 97, 128^3 260 -> 202, 240^3 1960 -> 1145; general
+// transient cells 32^3 97 -> 27, 97^3 207 -> 148, 256^3 2320 -> 2290.
+Q1Plan q1_plan(const Mesh &m, int ncu) {
+  Q1Plan plan;
+  if (!m.structured || (m.topo != TXA_HEX8 && m.topo != TXA_TET4)) return plan;
+  const int layers = m.nz + 1;
+  auto wide = [&](int slots, double *cost) {
+    const int gx = tiles_x(m, Wide::TX), gy = tiles_y(m, Wide::TY), tiles = gx * gy;
+    int nchunk = (kTargetBlocks + tiles - 1) / tiles;
+    nchunk = std::max(1, std::min(nchunk, (layers + 7) / 8));
+    int zc = (layers + nchunk - 1) / nchunk;
+    const int64_t limit = 4 * static_cast<int64_t>(slots);
+    if (static_cast<int64_t>(tiles) * ((layers + zc - 1) / zc) > limit) {
+      *cost = (static_cast<double>(tiles) * ((layers + zc - 1) / zc) / slots + 0.5) * (zc + 1.5);
+      return zc;
+    }
+    int last = 0;
+    *cost = 0.0;
+    for (int n = 1; n <= layers && (n == 1 || static_cast<int64_t>(tiles) * n <= limit); ++n) {
+      const int z = (layers + n - 1) / n;
+      if (z == last) continue;
+      last = z;
+      std::priority_queue<double, std::vector<double>, std::greater<double>> free_at;
+      double end = 0.0;
+      for (int k0 = 0; k0 < layers; k0 += z)
+        for (int t = 0; t < tiles; ++t) {
+          const int x = gx >= kYFastest ? t / gy : t % gx;   // tile_of_block's order
+          const double cols = std::min(Wide::TX - 1, m.nx + 1 - (Wide::TX - 1) * x) / double(Wide::TX - 1);
+          double at = 0.0;
+          if (static_cast<int>(free_at.size()) == slots) { at = free_at.top(); free_at.pop(); }
+          at += (std::min(z, layers - k0) + 1.5) * (0.5 + 0.5 * cols);
+          free_at.push(at);
+          end = std::max(end, at);
+        }
+      if (n == 1 || end < *cost) { *cost = end; zc = z; }
+    }
+    return zc;
+  };
+  auto small = [&](double *cost) {
+    const int64_t tiles = static_cast<int64_t>(tiles_x(m, Small::TX)) * tiles_y(m, Small::TY);
+    int zc = layers, last = 0;
+    *cost = 1e300;
+    for (int n = 1; n <= layers; ++n) {
+      const int z = (layers + n - 1) / n;
+      if (z == last) continue;
+      last = z;
+      const int64_t chunks = (layers + z - 1) / z;
+      double c = 1.05 * std::max(static_cast<double>(tiles * (layers + 2 * chunks)) / (2 * ncu) + 0.5 * (z + 2), z + 2.0);
+      if (tiles * chunks <= ncu) c = std::min(c, z + 1.0);
+      if (c < *cost) { *cost = c; zc = z; }
+    }
+    return zc;
+  };
+  double cw = 0.0, cs = 0.0, cf = 0.0;
+  const int zw = wide(ncu, &cw), zs = small(&cs);
+  plan.small = (m.topo == TXA_HEX8 && m.affine) || cs < cw;
+  plan.zc = plan.small ? zs : zw;
+  plan.zc_f = wide(2 * ncu, &cf);   // the residual kernel: two workgroups per CU by registers
+  return plan;
+}
+
 void launch_q1_hex8_diffusion(Mesh &m, const txa_assembly_args &a, hipStream_t s) {
-  // z slabs: enough workgroups to cover the 256 CUs several times over
-  const int gx = tiles_x(m), gy = tiles_y(m);
-  static_assert(NT == 512, "block shape");
-  int nchunk = (kTargetBlocks + gx * gy - 1) / (gx * gy);
-  nchunk = std::max(1, std::min(nchunk, (m.nz + 1 + 7) / 8));
-  int zc = (m.nz + 1 + nchunk - 1) / nchunk;
-  nchunk = (m.nz + 1 + zc - 1) / zc;
+  if (!a.f && !a.vals) return;
+  const int zc = a.vals ? m.q1.zc : m.q1.zc_f;
+  TXA_REQUIRE(zc > 0, TXA_ERR_LOGIC, "slab height missing (graph_build)");
+  const int nchunk = (m.nz + 1 + zc - 1) / zc;
   const Q1DiffParams p = make_params(m, a, zc);
-  dim3 grid(gx, gy, nchunk);
   const bool trans = a.transient != 0;
-  if (m.topo == TXA_TET4) launch_kind<TXA_TET4>(p, grid, a.precision, trans, s);
-  else if (m.affine) launch_kind<kHex8Affine>(p, grid, a.precision, trans, s);
-  else launch_kind<TXA_HEX8>(p, grid, a.precision, trans, s);
+  auto grid = [&](int tx, int ty) { return dim3(tiles_x(m, tx), tiles_y(m, ty), nchunk); };
+  if (!a.vals) {
+    const dim3 g = grid(Wide::TX, Wide::TY);
+    if (m.topo == TXA_TET4) launch_residual<TXA_TET4>(p, g, a.precision, trans, s);
+    else if (m.affine) launch_residual<kHex8Affine>(p, g, a.precision, trans, s);
+    else launch_residual<TXA_HEX8>(p, g, a.precision, trans, s);
+  } else if (m.q1.small) {
+    const dim3 g = grid(Small::TX, Small::TY);
+    if (m.topo == TXA_TET4) launch_kind<Small, TXA_TET4>(p, g, a.precision, trans, s);
+    else if (m.affine) launch_kind<Small, kHex8Affine>(p, g, a.precision, trans, s);
+    else launch_kind<Small, TXA_HEX8>(p, g, a.precision, trans, s);
+  } else {
+    const dim3 g = grid(Wide::TX, Wide::TY);
+    if (m.topo == TXA_TET4) launch_kind<Wide, TXA_TET4>(p, g, a.precision, trans, s);
+    else if (m.affine) launch_kind<Wide, kHex8Affine>(p, g, a.precision, trans, s);
+    else launch_kind<Wide, TXA_HEX8>(p, g, a.precision, trans, s);
+  }
   TXA_HIP(hipGetLastError());
 }
 
@@ -843,7 +1029,7 @@ struct Batch {
   int precision = TXA_FP64;
   bool transient = false;
   int slab = 0;   // vertex layers per work item (0: whole column)
-  int tx = kTX;   // tile width (vertex columns along x; the tile is tx x 256/tx)
+  int tx = Wide::TX;   // tile width (vertex columns along x; the tile is tx x 256/tx)
   int grid = 0;   // persistent workgroups
   std::vector<int> zc;
   std::vector<int4> items_h;   // hex8 items, then tet4 items
@@ -907,7 +1093,7 @@ void batch_build_items(Batch &b, int slab) {
     const int nch = (layers + zc - 1) / zc;
     std::vector<int4> &out = lists[m.topo == TXA_TET4 ? 1 : 0];
     for (int z = 0; z < nch; ++z)
-      for (int y = 0; y < tiles_y(m, b.tx); ++y)
+      for (int y = 0; y < tiles_y(m, Wide::NE / b.tx); ++y)
         for (int x = 0; x < tiles_x(m, b.tx); ++x) out.push_back(make_int4(static_cast<int>(i), x, y, z));
   }
   auto cost = [&](const int4 &w) {
@@ -980,22 +1166,22 @@ void batch_fill(Batch &b, const txa_assembly_args *args) {
   }
 }
 
-template <int TXV, int KIND>
+template <class T, int KIND>
 void launch_batch_tx(const Batch &b, dim3 g, const int4 *items, int n, BatchQueue *q, hipStream_t s) {
   if (b.precision == TXA_FP64) {
-    if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<TXV, KIND, double, true>), g, dim3(NT), 0, s, b.prm.p, items, n, q);
-    else hipLaunchKernelGGL((k_q1_batch_spec<TXV, KIND, double, false>), g, dim3(NT), 0, s, b.prm.p, items, n, q);
+    if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, double, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+    else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, double, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
   } else {
-    if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<TXV, KIND, float, true>), g, dim3(NT), 0, s, b.prm.p, items, n, q);
-    else hipLaunchKernelGGL((k_q1_batch_spec<TXV, KIND, float, false>), g, dim3(NT), 0, s, b.prm.p, items, n, q);
+    if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+    else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
   }
   TXA_HIP(hipGetLastError());
 }
 
 template <int KIND>
 void launch_batch(const Batch &b, dim3 g, const int4 *items, int n, BatchQueue *q, hipStream_t s) {
-  if (b.tx == 16) launch_batch_tx<16, KIND>(b, g, items, n, q, s);
-  else launch_batch_tx<32, KIND>(b, g, items, n, q, s);
+  if (b.tx == 16) launch_batch_tx<Square, KIND>(b, g, items, n, q, s);
+  else launch_batch_tx<Wide, KIND>(b, g, items, n, q, s);
 }
 
 void batch_enqueue(Batch &b, hipStream_t s, int *err) {
@@ -1014,9 +1200,9 @@ void batch_enqueue(Batch &b, hipStream_t s, int *err) {
     const int nall = static_cast<int>(b.items_h.size());
     const dim3 g(std::min(b.grid, nall));
     if (b.tx == 16)
-      hipLaunchKernelGGL((k_q1_batch_mixed<16, kHex8Affine, float, false>), g, dim3(NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
+      hipLaunchKernelGGL((k_q1_batch_mixed<Square, kHex8Affine, float, false>), g, dim3(Square::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
     else
-      hipLaunchKernelGGL((k_q1_batch_mixed<32, kHex8Affine, float, false>), g, dim3(NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
+      hipLaunchKernelGGL((k_q1_batch_mixed<Wide, kHex8Affine, float, false>), g, dim3(Wide::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
     TXA_HIP(hipGetLastError());
   }
   for (int k = 0; k < 2 && !b.mixed; ++k) {

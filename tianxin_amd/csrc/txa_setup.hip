@@ -618,6 +618,13 @@ void graph_build(Mesh &m, hipStream_t s) {
   }
   patch_build(m, s);   // node patches of single-block hex8 / tet4 meshes
   TXA_HIP(hipStreamSynchronize(s));
+  m.q1 = Q1Plan();
+  if (m.nfields == 1) {
+    int dev = 0, ncu = 0;
+    TXA_HIP(hipGetDevice(&dev));
+    TXA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    m.q1 = q1_plan(m, ncu);
+  }
   m.has_graph = true;
 }
 
