@@ -20,6 +20,7 @@
 #include <cstring>
 #include <functional>
 #include <queue>
+#include <type_traits>
 
 namespace txa {
 namespace {
@@ -38,7 +39,7 @@ struct Tile {
   static constexpr int NOWN = TX * (TY - 1);   // owner lanes with rows
 };
 using Wide = Tile<32, 256>;     // one workgroup per CU (LDS)
-using Square = Tile<16, 256>;   // one workgroup per CU, batches
+using Square = Tile<16, 256>;   // one workgroup per CU, FP64 batches
 using Small = Tile<16, 128>;    // two workgroups per CU
 using namespace q1elem;
 // element kinds of the lattice kernels: TXA_HEX8 (general trilinear cells), TXA_TET4 (six
@@ -1029,8 +1030,9 @@ struct Batch {
   int precision = TXA_FP64;
   bool transient = false;
   int slab = 0;   // vertex layers per work item (0: whole column)
-  int tx = Wide::TX;   // tile width (vertex columns along x; the tile is tx x 256/tx)
+  int tx = 16;    // tile width, vertex columns along x: 32 x 8; 16 x 16 (FP64), 16 x 8 (FP32)
   int grid = 0;   // persistent workgroups
+  int tile_y() const { return tx == 32 ? Wide::TY : precision == TXA_FP32 ? Small::TY : Square::TY; }
   std::vector<int> zc;
   std::vector<int4> items_h;   // hex8 items, then tet4 items
   size_t n_hex = 0;            // items of hex8 meshes (the first n_hex of items_h)
@@ -1093,7 +1095,7 @@ void batch_build_items(Batch &b, int slab) {
     const int nch = (layers + zc - 1) / zc;
     std::vector<int4> &out = lists[m.topo == TXA_TET4 ? 1 : 0];
     for (int z = 0; z < nch; ++z)
-      for (int y = 0; y < tiles_y(m, Wide::NE / b.tx); ++y)
+      for (int y = 0; y < tiles_y(m, b.tile_y()); ++y)
         for (int x = 0; x < tiles_x(m, b.tx); ++x) out.push_back(make_int4(static_cast<int>(i), x, y, z));
   }
   auto cost = [&](const int4 &w) {
@@ -1168,20 +1170,26 @@ void batch_fill(Batch &b, const txa_assembly_args *args) {
 
 template <class T, int KIND>
 void launch_batch_tx(const Batch &b, dim3 g, const int4 *items, int n, BatchQueue *q, hipStream_t s) {
-  if (b.precision == TXA_FP64) {
-    if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, double, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
-    else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, double, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
-  } else {
-    if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
-    else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+  if constexpr (!std::is_same<T, Small>::value) {   // Small: FP32 only
+    if (b.precision == TXA_FP64) {
+      if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, double, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+      else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, double, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+    }
+  }
+  if constexpr (!std::is_same<T, Square>::value) {   // Square: FP64 only
+    if (b.precision == TXA_FP32) {
+      if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+      else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+    }
   }
   TXA_HIP(hipGetLastError());
 }
 
 template <int KIND>
 void launch_batch(const Batch &b, dim3 g, const int4 *items, int n, BatchQueue *q, hipStream_t s) {
-  if (b.tx == 16) launch_batch_tx<Square, KIND>(b, g, items, n, q, s);
-  else launch_batch_tx<Wide, KIND>(b, g, items, n, q, s);
+  if (b.tx == 32) launch_batch_tx<Wide, KIND>(b, g, items, n, q, s);
+  else if (b.precision == TXA_FP32) launch_batch_tx<Small, KIND>(b, g, items, n, q, s);
+  else launch_batch_tx<Square, KIND>(b, g, items, n, q, s);
 }
 
 void batch_enqueue(Batch &b, hipStream_t s, int *err) {
@@ -1200,7 +1208,7 @@ void batch_enqueue(Batch &b, hipStream_t s, int *err) {
     const int nall = static_cast<int>(b.items_h.size());
     const dim3 g(std::min(b.grid, nall));
     if (b.tx == 16)
-      hipLaunchKernelGGL((k_q1_batch_mixed<Square, kHex8Affine, float, false>), g, dim3(Square::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
+      hipLaunchKernelGGL((k_q1_batch_mixed<Small, kHex8Affine, float, false>), g, dim3(Small::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
     else
       hipLaunchKernelGGL((k_q1_batch_mixed<Wide, kHex8Affine, float, false>), g, dim3(Wide::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
     TXA_HIP(hipGetLastError());
@@ -1262,8 +1270,26 @@ Batch *batch_create(const std::vector<Mesh *> &meshes, const std::vector<int> &i
   int dev = 0, ncu = 0;
   TXA_HIP(hipGetDevice(&dev));
   TXA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  b->grid = 2 * ncu;
-  batch_build_items(*b, 32);
+  // Shape until txa_batch_tune or txa_batch_shape sets another: width 16 (on 128 hex8 / tet4 meshes of
+  // 8-64 cells per axis 32 x 8 tiles take 661 us in FP32 and 765 in FP64, 16 x 8 two workgroups per
+  // CU 590 in FP32, 16 x 16 712 in FP64), the resident workgroups, and the slab height whose steps,
+  // one recomputed layer and the start of each item counted as two, spread over them with half a
+  // slab as tail, take least (4 meshes of 16-64 cells: 148 us with slabs of 32 layers, 100 with 6).
+  const int slots = precision == TXA_FP32 ? 2 * ncu : ncu;
+  b->grid = slots;
+  int slab = 0;
+  double best = 0.0;
+  for (int z : {4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+    double steps = 0.0, longest = 0.0;
+    for (const Mesh *m : meshes) {
+      const int layers = m->nz + 1, zc = std::min(z, layers), chunks = (layers + zc - 1) / zc;
+      steps += static_cast<double>(tiles_x(*m, b->tx)) * tiles_y(*m, b->tile_y()) * (layers + 2 * chunks);
+      longest = std::max(longest, zc + 2.0);
+    }
+    const double cost = std::max(steps / slots + 0.5 * longest, longest);
+    if (slab == 0 || cost < best) { best = cost; slab = z; }
+  }
+  batch_build_items(*b, slab);
   return b.release();
 }
 
@@ -1289,7 +1315,7 @@ void batch_assemble(Batch &b, const txa_assembly_args *args, bool use_graph, hip
   b.launched = true;
 }
 
-// Autotuner: times the batch over tile shapes (32 x 8, 16 x 16), slab heights (the
+// Autotuner: times the batch over tile widths (32, 16), slab heights (the
 // analogue of Panzer's workset size sweep) and persistent grid sizes, keeps the
 // fastest.  out: best ms.
 double batch_tune(Batch &b, const txa_assembly_args *args, hipStream_t s, int reps, int *err) {
