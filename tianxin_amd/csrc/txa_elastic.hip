@@ -1212,6 +1212,482 @@ __global__ __launch_bounds__(256, 4) void k_elastic8_affine(Elastic8Params p) {
   }
 }
 
+// General (trilinear) hex8 cells, three fields, FP64: node-centric assembly with no workspace.
+//
+// The element stiffness block of vertices a and b is T_ab = sum_q s_q g_a(q) g_b(q)^T over the
+// 2x2x2 Gauss points, with g_b(q) = C_q d_b(q) (C_q the cofactors of the point's Jacobian, d_b the
+// reference gradient) and s_q its weight over det^2.  Everything about a point's Jacobian is formed
+// once per (cell, point) and put in LDS; each lane then forms blocks of one row of the matrix.
+//
+// Signs and scales.  With J' the Jacobian from edge differences (hi - lo without their signs and
+// halves: dN_b/dxi_m = s_bm L L / 2, L = (1 +- 1/sqrt3)/2), a lane at point q sees
+// J = J' S_q / 2, S_q = diag of the point's signs, so J^-T dN_b = C' d(q ^ b) / det J' with
+// d(r)_x = sigma(r_x) L(r_y) L(r_z), sigma = +1 where point and vertex agree on the axis, -1 where
+// not, L the larger weight where they agree: the reference gradients depend on r = q ^ b only.
+constexpr double kLp = 0.78867513459481288225, kLm = 0.21132486540518711775;   // (1 +- 1/sqrt3) / 2
+constexpr int kPtStride = 12;   // doubles per (cell, point): C' (9), s, w |det J|, padding
+
+__device__ __forceinline__ constexpr double gL(int r) { return r ? kLm : kLp; }
+__device__ __forceinline__ constexpr double gS(int r) { return r ? -1.0 : 1.0; }
+
+// Lane t of a group of eight <-> corner bits: z = t >> 2, (x, y) = (t & 3), complemented where z = 1,
+// so that the neighbour along x, y, z is lane t ^ 1, t ^ 2, t ^ 7: one DPP move each.
+__device__ __forceinline__ int corner_of_lane(int t) { return (t & 4) ? (t ^ 3) : t; }
+
+template <int AXIS>
+__device__ __forceinline__ double corner_swap(double x) {
+  return dpp_f64<AXIS == 0 ? 0xB1 : (AXIS == 1 ? 0x4E : 0x141), 0xf>(x);
+}
+
+// J' at this lane's point from this lane's corner value of one coordinate (eight lanes per cell).
+__device__ __forceinline__ void corner_grad(double X, double &gx, double &gy, double &gz) {
+  const double px = corner_swap<0>(X);
+  const double ex = X - px, ix = kLp * X + kLm * px;
+  const double py = corner_swap<1>(ix), pe = corner_swap<1>(ex);
+  const double ey = ix - py, iy = kLp * ix + kLm * py, exy = kLp * ex + kLm * pe;
+  const double pz = corner_swap<2>(iy), p0 = corner_swap<2>(exy), p1 = corner_swap<2>(ey);
+  gz = iy - pz;
+  gx = kLp * exy + kLm * p0;
+  gy = kLp * ey + kLm * p1;
+}
+
+// The point table entry of this lane: corner coordinates in, C', s and w |det J| out.
+// (ok false: a cell outside the mesh, whose point weights are zero.)
+__device__ __forceinline__ void point_entry(double X, double Y, double Z, int t, bool ok, double *tab) {
+  double J[3][3];
+  corner_grad(X, J[0][0], J[0][1], J[0][2]);
+  corner_grad(Y, J[1][0], J[1][1], J[1][2]);
+  corner_grad(Z, J[2][0], J[2][1], J[2][2]);
+  double C[9];
+  C[0] = J[1][1] * J[2][2] - J[1][2] * J[2][1];
+  C[1] = J[1][2] * J[2][0] - J[1][0] * J[2][2];
+  C[2] = J[1][0] * J[2][1] - J[1][1] * J[2][0];
+  C[3] = J[0][2] * J[2][1] - J[0][1] * J[2][2];
+  C[4] = J[0][0] * J[2][2] - J[0][2] * J[2][0];
+  C[5] = J[0][1] * J[2][0] - J[0][0] * J[2][1];
+  C[6] = J[0][1] * J[1][2] - J[0][2] * J[1][1];
+  C[7] = J[0][2] * J[1][0] - J[0][0] * J[1][2];
+  C[8] = J[0][0] * J[1][1] - J[0][1] * J[1][0];
+  const double det = J[0][0] * C[0] + J[0][1] * C[1] + J[0][2] * C[2];
+  const int q = corner_of_lane(t);
+  // sign of S_q: an odd number of low sides is negative; the true determinant is det * S_q / 8, and
+  // the measure takes the sign of the first point's (Intrepid2 computeCellMeasure)
+  const double s8 = (__popc(q) & 1) ? 0.125 : -0.125;
+  const int hi = __double2hiint(det * s8);
+  int h0 = __builtin_amdgcn_update_dpp(0, hi, 0x00, 0xf, 0xf, false);    // lanes 0-3: lane 0's
+  const int h1 = __builtin_amdgcn_update_dpp(0, h0, 0x141, 0xf, 0xf, false);   // lanes 4-7: lane 3's copy
+  h0 = (t & 4) ? h1 : h0;
+  const double w = ok ? (h0 < 0 ? -s8 : s8) : 0.0;
+  double id = __builtin_amdgcn_rcp(det);   // 1 / det to within an ulp: two Newton steps
+  id = __builtin_fma(__builtin_fma(-det, id, 1.0), id, id);
+  id = __builtin_fma(__builtin_fma(-det, id, 1.0), id, id);
+  double2 *o = reinterpret_cast<double2 *>(tab + q * kPtStride);
+  o[0] = make_double2(C[0], C[1]);
+  o[1] = make_double2(C[2], C[3]);
+  o[2] = make_double2(C[4], C[5]);
+  o[3] = make_double2(C[6], C[7]);
+  o[4] = make_double2(C[8], ok ? w * id : 0.0);
+  o[5] = make_double2(w * det, 0.0);
+}
+
+// Blocks T_ab (and mass sums) of one row vertex a and NBL = 2^NX vertices b that differ in their
+// first NX axes (index k of block: corner bits bb ^ k on those axes, bb the lane's base corner), over
+// the eight points of the lane's cell.  fa = a ^ bb.  m0 = sum_q w |det| N_a.
+template <int NX, bool TR>
+__device__ __forceinline__ void row_blocks(const double *tab, int bb, int fa, double (&T)[1 << NX][3][3],
+                                           double (&M)[1 << NX], double &m0) {
+  constexpr int NBL = 1 << NX;
+  // of vertex a along each axis at the point on base corner bb's side (0) and the other (1)
+  const bool ax = fa & 1, ay = fa & 2, az = fa & 4;
+  const double Lx[2] = {ax ? kLm : kLp, ax ? kLp : kLm}, Ly[2] = {ay ? kLm : kLp, ay ? kLp : kLm},
+               Lz[2] = {az ? kLm : kLp, az ? kLp : kLm};
+  const double sx = ax ? -1.0 : 1.0, sy = ay ? -1.0 : 1.0, sz = az ? -1.0 : 1.0;
+  double YZ[2][2], XZ[2][2], XY[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      YZ[i][j] = sx * Ly[i] * Lz[j];
+      XZ[i][j] = sy * Lx[i] * Lz[j];
+      XY[i][j] = sz * Lx[i] * Ly[j];
+    }
+  const double Lzs[2] = {sz * Lz[0], sz * Lz[1]};
+#pragma unroll
+  for (int k = 0; k < NBL; ++k) {
+    M[k] = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) T[k][i][j] = 0.0;
+  }
+  m0 = 0.0;
+#pragma unroll
+  for (int kq = 0; kq < 8; ++kq) {
+    const int qx = kq & 1, qy = (kq >> 1) & 1, qz = kq >> 2;   // the point relative to corner bb
+    const double2 *o = reinterpret_cast<const double2 *>(tab + (bb ^ kq) * kPtStride);
+    const double2 c0 = o[0], c1 = o[1], c2 = o[2], c3 = o[3], c4 = o[4];
+    const double C[3][3] = {{c0.x, c0.y, c1.x}, {c1.y, c2.x, c2.y}, {c3.x, c3.y, c4.x}};
+    const double mu = o[5].x * XY[qx][qy] * Lzs[qz];   // w |det| N_a
+    const double dx = gS(qx) * c4.y * YZ[qy][qz], dy = gS(qy) * c4.y * XZ[qx][qz], dz = gS(qz) * c4.y * XY[qx][qy];
+    double v[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] = C[i][0] * dx + C[i][1] * dy + C[i][2] * dz;
+    m0 += mu;
+#pragma unroll
+    for (int k = 0; k < NBL; ++k) {
+      const int rx = qx ^ (k & 1), ry = NX > 1 ? qy ^ ((k >> 1) & 1) : qy, rz = qz;
+      double g[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        g[j] = C[j][0] * (gS(rx) * gL(ry) * gL(rz)) + C[j][1] * (gL(rx) * gS(ry) * gL(rz)) +
+               C[j][2] * (gL(rx) * gL(ry) * gS(rz));
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) T[k][i][j] += v[i] * g[j];
+      if (TR) M[k] += mu * (gL(rx) * gL(ry) * gL(rz));
+    }
+    // one point's data in registers at a time: the next point's address waits for these sums (left
+    // to itself the compiler loads all eight points first and spills)
+#pragma unroll
+    for (int k = 0; k < NBL; ++k)
+      asm volatile("" : "+v"(bb), "+v"(T[k][0][0]), "+v"(T[k][0][1]), "+v"(T[k][0][2]), "+v"(T[k][1][0]), "+v"(T[k][1][1]),
+                   "+v"(T[k][1][2]), "+v"(T[k][2][0]), "+v"(T[k][2][1]), "+v"(T[k][2][2]), "+v"(M[k]));
+  }
+}
+
+// One workgroup: 4 x 4 nodes of one lattice plane, a wave per line of four nodes along x, 16 lanes
+// per node: lane (cell c around the node, half h) forms the blocks of the four vertices of c on its
+// low / high z side.  The 5 x 5 x 2 cells' points are formed once for the 16 nodes (50 cells instead
+// of 128).  Blocks of different cells that meet in one neighbour are summed by DPP moves along x, y,
+// z in that order, one lane then writes each neighbour's block into the row buffer (which lies over
+// the point table) and the wave stores the rows, its four nodes as one range where their LIDs follow
+// each other.  Every sum has a fixed order: results are bitwise reproducible.
+struct Elastic8GParams {
+  Elastic8Params p;
+  const double *X, *Y, *Z;
+};
+
+constexpr int kN8 = 4;                                      // nodes along x and y per workgroup
+constexpr int kV8 = (kN8 + 2) * (kN8 + 2) * 3;              // staged vertices
+constexpr int kC8 = (kN8 + 1) * (kN8 + 1) * 2;              // cells
+constexpr int kRow8 = 3 * 81;                               // entries of a node's rows at most
+
+template <bool TR>
+__global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp) {
+  const Elastic8Params &p = gp.p;
+  __shared__ __align__(16) double tab[kC8 * 8 * kPtStride];   // points; then the rows of the 16 nodes
+  __shared__ double vtx[TR ? 9 : 6][kV8];                            // x, y, z, u + b_R v, a_R v + a
+  static_assert(kN8 * kN8 * kRow8 <= kC8 * 8 * kPtStride, "rows fit over the point table");
+  int tid = threadIdx.x;
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // lane of a node = ox ^ 2 oy ^ 8 oz ^ 15 h: the partner cell along x is lane ^ 1, along y lane ^ 2,
+  // and the (upper cell, low half) of lanes 8-11 meets the (lower cell, high half) of lanes 12-15
+  // at lane ^ 7: one DPP move each
+  const int l16 = lane & 15, lu = (l16 & 4) ? l16 ^ 15 : l16;
+  const int n = lane >> 4, h = (l16 >> 2) & 1, ox = lu & 1, oy = (lu >> 1) & 1, oz = lu >> 3;
+  const int sx = p.nx + 1, sxy = sx * (p.ny + 1);
+  const int gx = (sx + kN8 - 1) / kN8, gy = (p.ny + 1 + kN8 - 1) / kN8;
+  const int ntile = gx * gy * (p.nz + 1);
+  const bool tra = TR && p.xddot;
+  const double lamf = p.nu / ((1.0 + p.nu) * (1.0 - 2.0 * p.nu)), muf = 0.5 / (1.0 + p.nu);
+  const double cK = TR ? p.beta + p.alpha * p.rb : p.beta;
+  const double cM = TR ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
+  for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+    asm volatile("" : "+v"(tid));   // the staging indices are formed per tile, not kept in registers
+    const int I0 = tile % gx * kN8, J0 = tile / gx % gy * kN8, K = tile / (gx * gy);
+    // vertices (clamped into the mesh: what lies outside belongs to no cell of the mesh)
+    if (tid < kV8) {
+      const int vx = min(max(I0 - 1 + tid % (kN8 + 2), 0), p.nx);
+      const int vy = min(max(J0 - 1 + tid / (kN8 + 2) % (kN8 + 2), 0), p.ny);
+      const int vz = min(max(K - 1 + tid / ((kN8 + 2) * (kN8 + 2)), 0), p.nz);
+      const int vi = vx + sx * vy + sxy * vz;
+      const int32_t L = p.point_lid[3 * vi];
+      vtx[0][tid] = gp.X[vi];
+      vtx[1][tid] = gp.Y[vi];
+      vtx[2][tid] = gp.Z[vi];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const double u = p.x[L + j];
+        if constexpr (TR) {
+          const double v = p.xdot[L + j], a = tra ? p.xddot[L + j] : 0.0;
+          vtx[3 + j][tid] = u + p.rb * v;
+          vtx[6 + j][tid] = p.ra * v + a;
+        } else {
+          vtx[3 + j][tid] = u;
+        }
+      }
+    }
+    // this lane's node and cell: their loads go out before the barrier
+    const int I = I0 + n, Jy = J0 + w;
+    const bool node_ok = I <= p.nx && Jy <= p.ny;
+    const int nodev = min(I, p.nx) + sx * min(Jy, p.ny) + sxy * K;
+    const int32_t L0 = p.point_lid[3 * nodev];
+    const int cx = I - 1 + ox, cy = Jy - 1 + oy, cz = K - 1 + oz;
+    const bool cell_ok = node_ok && cx >= 0 && cx < p.nx && cy >= 0 && cy < p.ny && cz >= 0 && cz < p.nz;
+    const double E = p.coef[cell_ok ? cx + p.nx * (cy + p.ny * cz) : 0];
+    __syncthreads();
+    // points of the cells
+#pragma unroll 1
+    for (int task = tid; task < kC8 * 8; task += 256) {
+      const int c = task >> 3, t = task & 7, b = corner_of_lane(t);
+      const int lx = c % (kN8 + 1), ly = c / (kN8 + 1) % (kN8 + 1), lz = c / ((kN8 + 1) * (kN8 + 1));
+      const int vi = lx + (b & 1) + (kN8 + 2) * (ly + ((b >> 1) & 1) + (kN8 + 2) * (lz + (b >> 2)));
+      const bool ok = static_cast<unsigned>(I0 - 1 + lx) < static_cast<unsigned>(p.nx) &&
+                      static_cast<unsigned>(J0 - 1 + ly) < static_cast<unsigned>(p.ny) &&
+                      static_cast<unsigned>(K - 1 + lz) < static_cast<unsigned>(p.nz);
+      point_entry(vtx[0][vi], vtx[1][vi], vtx[2][vi], t, ok, tab + c * 8 * kPtStride);
+    }
+    const int64_t base = p.rowptr[L0];
+    const int len = min(static_cast<int>(p.rowptr[L0 + 1] - base), 81);
+    const uint16_t *np = p.nperm + static_cast<int64_t>(L0 / 3) * p.nperm_w;
+    // neighbour slot of block k: dx = 0 where k complements the cell's side, -1 / +1 otherwise
+    int pos[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int dx = (k & 1) ? 1 : 2 * ox, dy = (k & 2) ? 1 : 2 * oy, dz = oz + h;
+      pos[k] = np[dx + 3 * dy + 9 * dz];
+    }
+    __syncthreads();
+    double T[4][3][3], M[4], m0;
+    const int bb = ox + 2 * oy + 4 * h;           // base corner: the cell's far side, half h
+    const int av = (1 - ox) + 2 * (1 - oy) + 4 * (1 - oz);
+    const int cl = (n + ox) + (kN8 + 1) * (w + oy + (kN8 + 1) * oz);
+    row_blocks<2, TR>(tab + cl * 8 * kPtStride, bb, av ^ bb, T, M, m0);
+    const double lam = cell_ok ? E * lamf : 0.0, mu = cell_ok ? E * muf : 0.0;
+    double rr[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int bx = ox ^ (k & 1), by = oy ^ (k >> 1);
+      const int vi = (n + ox + bx) + (kN8 + 2) * ((w + oy + by) + (kN8 + 2) * (oz + h));
+      const double trs = T[k][0][0] + T[k][1][1] + T[k][2][2];
+      const double Mab = TR ? p.rho * M[k] : 0.0;
+      double ut[3], mt[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) { ut[j] = vtx[3 + j][vi]; mt[j] = TR ? vtx[TR ? 6 + j : 0][vi] : 0.0; }
+      double t9[3][3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) t9[i][j] = T[k][i][j];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const double Kv = lam * t9[i][j] + mu * t9[j][i] + (i == j ? mu * trs : 0.0);
+          rr[i] += Kv * ut[j];
+          double jv = cK * Kv;
+          if (TR && i == j) {
+            jv += cM * Mab;
+            rr[i] += Mab * mt[j];
+          }
+          T[k][i][j] = jv;
+        }
+    }
+    // residual: the cell's source load enters once, then the sum over the node's 16 lanes
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      double r = rr[i] - (h == 0 ? p.src[i] * m0 : 0.0);
+      r += dpp_f64<0xB1, 0xf>(r);
+      r += dpp_f64<0x4E, 0xf>(r);
+      r += dpp_f64<0x141, 0xf>(r);
+      r += dpp_f64<0x140, 0xf>(r);
+      rr[i] = r;
+    }
+    if (p.f && node_ok && l16 < 3) p.f[L0 + l16] = l16 == 0 ? rr[0] : (l16 == 1 ? rr[1] : rr[2]);
+    if (p.vals) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            double v = T[k][i][j];
+            if (k & 1) v += dpp_f64<0xB1, 0xf>(v);   // the cells on both sides along x
+            if (k & 2) v += dpp_f64<0x4E, 0xf>(v);   // along y
+            const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x141, 0xf, 0xc, false);
+            const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x141, 0xf, 0xc, false);
+            T[k][i][j] = v + __hiloint2double(hi, lo);   // along z (lanes 8-15)
+          }
+    }
+    __syncthreads();   // every wave is done with the points and the vertices: the rows go over the points
+    if (p.vals) {
+      // the rows of the wave's nodes, one after another as in the matrix where their LIDs are
+      const int64_t base0 = __shfl(base, 0);
+      const int32_t L00 = __shfl(L0, 0);
+      const bool run = __all(!node_ok || L0 == L00 + 3 * n);
+      double *rows = tab + w * kN8 * kRow8;
+      double *mine = rows + (run ? static_cast<int>(base - base0) : n * kRow8);
+      const bool zown = (oz == h) || h;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (node_ok && pos[k] + 2 < len && zown && !((k & 1) && ox) && !((k & 2) && oy)) {
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) mine[i * len + pos[k] + j] = T[k][i][j];
+        }
+      }
+      gather_lds_sync();
+      const int nok = min(kN8, sx - I0);   // nodes of the line inside the mesh
+      if (Jy <= p.ny) {
+        if (run) {
+          const int last = 16 * (nok - 1);
+          const int total = static_cast<int>(__shfl(base, last) - base0) + 3 * __shfl(len, last);
+          row_store(rows, p.vals + base0, total, lane);
+        } else {
+          for (int m = 0; m < nok; ++m) {
+            const int64_t bm = __shfl(base, 16 * m);
+            row_store(rows + m * kRow8, p.vals + bm, 3 * __shfl(len, 16 * m), lane);
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// The same row blocks on an uploaded hex8 mesh (one block): one wave per two nodes (LIDs 3 n, 3 n + 1,
+// 3 n + 2), 32 lanes per node: lane (element instance c of eight at a time, corner y and z) forms the
+// blocks of the two vertices along x.  Instances come from the node's list (ascending), the row
+// positions from their slot maps; the blocks are added into the node's rows in LDS instance by
+// instance, so the sums have a fixed order, and the rows are stored once.
+struct Elastic8UParams {
+  Elastic8Params p;
+  const double *X, *Y, *Z;
+  int64_t nnodes;
+  const int64_t *conn;      // [E][8] vertex ids
+  const int32_t *elem_lid;  // [E][24]
+  const int64_t *occ_ptr;   // [nnodes + 1]
+  const int32_t *occ;       // e * 8 + a per instance
+  const uint16_t *slot;     // [instances][8]
+};
+
+template <bool TR>
+__global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
+  const Elastic8Params &p = gp.p;
+  __shared__ __align__(16) double tab[2 * 8 * 8 * kPtStride];
+  __shared__ double rows[2][kRow8];
+  const int lane = threadIdx.x;
+  const int n = lane >> 5, c = (lane >> 2) & 7, bb = (lane & 3) << 1;   // base corner (0, y, z)
+  const int t = lane & 7, tb = corner_of_lane(t);
+  const int ts = tb ^ ((tb >> 1) & 1);   // binary corner -> element vertex order (its own inverse)
+  const bool tra = TR && p.xddot;
+  const double lamf = p.nu / ((1.0 + p.nu) * (1.0 - 2.0 * p.nu)), muf = 0.5 / (1.0 + p.nu);
+  const double cK = TR ? p.beta + p.alpha * p.rb : p.beta;
+  const double cM = TR ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
+  const int64_t npair = (gp.nnodes + 1) / 2;
+  for (int64_t pair = blockIdx.x; pair < npair; pair += gridDim.x) {
+    const int64_t node0 = 2 * pair, node = min(node0 + n, gp.nnodes - 1);
+    const bool node_ok = node0 + n < gp.nnodes;
+    // instance ranges of both nodes (wave-uniform) and of this lane's
+    const int64_t r0 = gp.occ_ptr[node0], r1 = gp.occ_ptr[node0 + 1];
+    const int64_t r2 = gp.occ_ptr[min(node0 + 2, gp.nnodes)];
+    const int64_t first = n ? r1 : r0;
+    const int cnt = node_ok ? static_cast<int>((n ? r2 : r1) - first) : 0;
+    const int most = max(static_cast<int>(r1 - r0), static_cast<int>(r2 - r1));
+    const int32_t L0 = static_cast<int32_t>(3 * node);
+    const int64_t base = p.rowptr[L0];
+    const int len = min(static_cast<int>(p.rowptr[L0 + 1] - base), 81);
+    if (p.vals)
+      for (int k = lane; k < 2 * kRow8; k += 64) (&rows[0][0])[k] = 0.0;
+    double racc[3] = {0.0, 0.0, 0.0};
+    for (int g = 0; g < most; g += 8) {
+      // points: eight lanes per instance, node 0's instances, then node 1's
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const int64_t lo = m ? r1 : r0, hi = m ? r2 : r1;
+        const int64_t k = lo + g + (lane >> 3);
+        const bool ok = k < hi;
+        const int64_t e = ok ? gp.occ[k] >> 3 : 0;
+        const int64_t v = gp.conn[8 * e + ts];
+        point_entry(gp.X[v], gp.Y[v], gp.Z[v], t, ok, tab + (m * 8 + (lane >> 3)) * 8 * kPtStride);
+      }
+      // this lane's instance, its modulus, vertices' state and row positions
+      const bool ok = g + c < cnt;
+      const int64_t k = ok ? first + g + c : r0;
+      const int32_t occ = gp.occ[k];
+      const int64_t e = occ >> 3;
+      const int as = occ & 7, av = as ^ ((as >> 1) & 1);
+      const double E = p.coef[e];
+      double ut[2][3], mt[2][3];
+      int pos[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int bs = (bb | b) ^ ((bb >> 1) & 1);
+        const int32_t L = gp.elem_lid[(8 * e + bs) * 3];
+        pos[b] = gp.slot[8 * k + bs];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          ut[b][j] = p.x[L + j];
+          mt[b][j] = 0.0;
+          if constexpr (TR) {
+            const double v = p.xdot[L + j], a = tra ? p.xddot[L + j] : 0.0;
+            ut[b][j] += p.rb * v;
+            mt[b][j] = p.ra * v + a;
+          }
+        }
+      }
+      gather_lds_sync();
+      double T[2][3][3], M[2], m0;
+      row_blocks<1, TR>(tab + (n * 8 + c) * 8 * kPtStride, bb, av ^ bb, T, M, m0);
+      const double lam = ok ? E * lamf : 0.0, mu = ok ? E * muf : 0.0;
+      if (!ok) m0 = 0.0;
+      double rr[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const double trs = T[b][0][0] + T[b][1][1] + T[b][2][2];
+        const double Mab = TR ? p.rho * M[b] : 0.0;
+        double t9[3][3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) t9[i][j] = T[b][i][j];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const double Kv = lam * t9[i][j] + mu * t9[j][i] + (i == j ? mu * trs : 0.0);
+            rr[i] += Kv * ut[b][j];
+            double jv = cK * Kv;
+            if (TR && i == j) {
+              jv += cM * Mab;
+              rr[i] += Mab * mt[b][j];
+            }
+            T[b][i][j] = jv;
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) racc[i] += ok ? rr[i] - (bb == 0 ? p.src[i] * m0 : 0.0) : 0.0;
+      if (p.vals) {
+        // one wave's LDS operations execute in order and the lanes of one step hit distinct entries:
+        // every entry is summed in instance order
+#pragma unroll
+        for (int cc = 0; cc < 8; ++cc)
+          if (c == cc && ok)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+              if (pos[b] + 2 < len)
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+#pragma unroll
+                  for (int j = 0; j < 3; ++j) atomicAdd(&rows[n][i * len + pos[b] + j], T[b][i][j]);
+      }
+      gather_lds_sync();   // the points are read; the next eight instances go over them
+    }
+    // residual over the node's 32 lanes (the total ends in the second row of 16), rows
+#pragma unroll
+    for (int i = 0; i < 3; ++i) racc[i] = group_sum<32>(racc[i]);
+    const int l32 = lane & 31;
+    if (p.f && node_ok && l32 >= 16 && l32 < 19) p.f[L0 + l32 - 16] = l32 == 16 ? racc[0] : (l32 == 17 ? racc[1] : racc[2]);
+    if (p.vals) {
+      for (int m = 0; m < 2 && node0 + m < gp.nnodes; ++m)
+        row_store(rows[m], p.vals + __shfl(base, 32 * m), 3 * __shfl(len, 32 * m), lane);
+      gather_lds_sync();
+    }
+  }
+}
+
 template <int NB, int NQ, int BS, int MODE>
 void launch(const ElasticParams &p, hipStream_t s) {
   int dev = 0, ncu = 0;
@@ -1235,6 +1711,13 @@ size_t ws_round(size_t b) { return (b + kWsAlign - 1) / kWsAlign * kWsAlign; }
 // affine HEX8 bricks take the node-centric kernel (no workspace) in every precision
 bool affine_hex8(const Mesh &m) {
   return m.topo == TXA_HEX8 && m.affine && m.structured && m.nfields == 3 && m.npoints < (int64_t(1) << 31);
+}
+
+// hex8 elasticity on general cells in FP64: the node kernels on bricks and on uploads whose
+// rows fit them
+bool general_hex8(const Mesh &m, int precision) {
+  if (m.topo != TXA_HEX8 || m.nfields != 3 || precision != TXA_FP64) return false;
+  return m.structured ? !m.affine && m.npoints < (int64_t(1) << 31) : m.uocc.p != nullptr;
 }
 
 // Streams and events of the element / gather slab pipeline, one set per host thread and device
@@ -1348,33 +1831,74 @@ void node_perm_build(Mesh &m, hipStream_t s) {
   }
 }
 
+namespace {
+
+Elastic8Params elastic8_params(const Mesh &m, const txa_assembly_args &a) {
+  Elastic8Params q;
+  q.nx = m.nx; q.ny = m.ny; q.nz = m.nz;
+  q.npoints = m.npoints;
+  q.point_lid = m.point_lid.p;
+  q.rowptr = m.rowptr.p;
+  q.nperm = m.nperm.p;
+  q.nperm_w = m.nperm_w;
+  q.geom = m.cell_geom.p;
+  q.coef = a.coef;
+  q.nu = a.nu; q.rho = a.rho;
+  q.src[0] = a.src[0]; q.src[1] = a.src[1]; q.src[2] = a.src[2];
+  q.ra = a.rayleigh_a; q.rb = a.rayleigh_b;
+  q.x = a.x; q.xdot = a.xdot; q.xddot = a.xddot;
+  q.alpha = a.alpha; q.beta = a.beta; q.gamma2 = a.gamma2;
+  q.transient = a.transient;
+  q.f = a.f; q.vals = a.vals;
+  return q;
+}
+
+// workgroups for a grid-stride kernel: the resident ones, or as many as there are items
+template <class Kernel>
+unsigned resident_grid(Kernel k, int64_t items, int threads = 256) {
+  int dev = 0, ncu = 0, per_cu = 0;
+  TXA_HIP(hipGetDevice(&dev));
+  TXA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  TXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, 0));
+  const int64_t want = static_cast<int64_t>(ncu) * std::max(per_cu, 1);
+  return static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(items, want)));
+}
+
+}  // namespace
+
 void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws) {
   if (!a.f && !a.vals) return;
   if (affine_hex8(m)) {
     TXA_REQUIRE(m.cell_geom.p != nullptr, TXA_ERR_LOGIC, "cell geometry missing (graph_build)");
-    Elastic8Params q;
-    q.nx = m.nx; q.ny = m.ny; q.nz = m.nz;
-    q.npoints = m.npoints;
-    q.point_lid = m.point_lid.p;
-    q.rowptr = m.rowptr.p;
-    q.nperm = m.nperm.p;
-    q.nperm_w = m.nperm_w;
-    q.geom = m.cell_geom.p;
-    q.coef = a.coef;
-    q.nu = a.nu; q.rho = a.rho;
-    q.src[0] = a.src[0]; q.src[1] = a.src[1]; q.src[2] = a.src[2];
-    q.ra = a.rayleigh_a; q.rb = a.rayleigh_b;
-    q.x = a.x; q.xdot = a.xdot; q.xddot = a.xddot;
-    q.alpha = a.alpha; q.beta = a.beta; q.gamma2 = a.gamma2;
-    q.transient = a.transient;
-    q.f = a.f; q.vals = a.vals;
-    int dev = 0, ncu = 0, per_cu = 0;
-    TXA_HIP(hipGetDevice(&dev));
-    TXA_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    TXA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_elastic8_affine, 256, 0));
-    const int64_t want = static_cast<int64_t>(ncu) * std::max(per_cu, 1);
-    const unsigned grid = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>((m.npoints + 3) / 4, want)));
-    hipLaunchKernelGGL(k_elastic8_affine, dim3(grid), dim3(256), 0, s, q);
+    const Elastic8Params q = elastic8_params(m, a);
+    hipLaunchKernelGGL(k_elastic8_affine, dim3(resident_grid(k_elastic8_affine, (m.npoints + 3) / 4)), dim3(256), 0, s, q);
+    TXA_HIP(hipGetLastError());
+    return;
+  }
+  if (general_hex8(m, a.precision) && m.structured) {
+    Elastic8GParams q;
+    q.p = elastic8_params(m, a);
+    q.X = m.xyz.p; q.Y = m.xyz.p + m.nverts; q.Z = m.xyz.p + 2 * m.nverts;
+    const int64_t tiles = static_cast<int64_t>((m.nx + 1 + kN8 - 1) / kN8) * ((m.ny + 1 + kN8 - 1) / kN8) * (m.nz + 1);
+    if (a.transient && a.xdot)
+      hipLaunchKernelGGL(k_elastic8_general<true>, dim3(resident_grid(k_elastic8_general<true>, tiles)), dim3(256), 0, s, q);
+    else
+      hipLaunchKernelGGL(k_elastic8_general<false>, dim3(resident_grid(k_elastic8_general<false>, tiles)), dim3(256), 0, s, q);
+    TXA_HIP(hipGetLastError());
+    return;
+  }
+  if (general_hex8(m, a.precision)) {
+    Elastic8UParams q;
+    q.p = elastic8_params(m, a);
+    q.X = m.xyz.p; q.Y = m.xyz.p + m.nverts; q.Z = m.xyz.p + 2 * m.nverts;
+    q.nnodes = m.ndofs / 3;
+    q.conn = m.conn.p; q.elem_lid = m.elem_lid.p;
+    q.occ_ptr = m.uocc_ptr.p; q.occ = m.uocc.p; q.slot = m.uslot.p;
+    const int64_t pairs = (q.nnodes + 1) / 2;
+    if (a.transient && a.xdot)
+      hipLaunchKernelGGL(k_elastic8_upload<true>, dim3(resident_grid(k_elastic8_upload<true>, pairs, 64)), dim3(64), 0, s, q);
+    else
+      hipLaunchKernelGGL(k_elastic8_upload<false>, dim3(resident_grid(k_elastic8_upload<false>, pairs, 64)), dim3(64), 0, s, q);
     TXA_HIP(hipGetLastError());
     return;
   }
