@@ -943,14 +943,15 @@ static size_t gather_ke_doubles(const Mesh &m, std::vector<int64_t> *begin) {
 
 // Workspace of the structured kernels' own parts (the elasticity blocks), before the
 // staging arrays of an accumulating call.
-static size_t kernel_workspace_bytes(const Mesh &m, int physics, int precision, bool want_f, bool want_vals) {
+static size_t kernel_workspace_bytes(const Mesh &m, int physics, int precision, bool want_f, bool want_vals,
+                                     bool footprint = false) {
   if (patch_supported(m, physics, precision)) return patch_workspace_bytes(m);
   if (lane_gather_mesh(m, physics, precision)) return want_vals ? sizeof(double) * gather_ke_doubles(m, nullptr) : 0;
   txa_assembly_args a{};
   a.physics = physics;
   a.precision = precision;
   if (uses_q1_path(m, physics, precision) || !elastic_supported(m, a)) return 0;
-  return elastic_workspace_bytes(m, precision, want_f, want_vals);
+  return elastic_workspace_bytes(m, precision, want_f, want_vals, footprint);
 }
 
 static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
@@ -965,8 +966,8 @@ static bool stages_rows(const Mesh &m, int physics, int precision, bool accumula
 }
 
 size_t assemble_workspace_bytes(const Mesh &m, int physics, int precision, bool want_f, bool want_vals,
-                                bool accumulate) {
-  size_t b = round256(kernel_workspace_bytes(m, physics, precision, want_f, want_vals));
+                                bool accumulate, bool footprint) {
+  size_t b = round256(kernel_workspace_bytes(m, physics, precision, want_f, want_vals, footprint));
   if (stages_rows(m, physics, precision, accumulate))
     b += (want_f ? round256(sizeof(double) * m.ndofs) : 0) + (want_vals ? round256(sizeof(double) * m.nnz) : 0);
   return b;

@@ -327,7 +327,7 @@ int txa_assemble_noalloc(txa_ctx ctx, int mesh_id, const txa_assembly_args *args
     TXA_REQUIRE(args, TXA_ERR_INVALID, "null args");
     Mesh &m = ctx->mesh(mesh_id);
     const size_t wsb = txa::assemble_workspace_bytes(m, args->physics, args->precision, args->f != nullptr,
-                                                     args->vals != nullptr, args->accumulate != 0);
+                                                     args->vals != nullptr, args->accumulate != 0, true);
     TXA_REQUIRE(wsb <= kScratchBytes, TXA_ERR_NOMEM,
                 "txa_assemble_noalloc: this assembly needs " + std::to_string(wsb) +
                     " bytes of workspace; the static workspace holds " + std::to_string(kScratchBytes) +

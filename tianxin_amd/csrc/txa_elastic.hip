@@ -1363,6 +1363,10 @@ __device__ __forceinline__ void row_blocks(const double *tab, int bb, int fa, do
 // z in that order, one lane then writes each neighbour's block into the row buffer (which lies over
 // the point table) and the wave stores the rows, its four nodes as one range where their LIDs follow
 // each other.  Every sum has a fixed order: results are bitwise reproducible.
+// Bound by VALU issue (about 520 instructions per node, 65% busy at two workgroups per CU, 208
+// VGPRs; held to 168 for three it spills and takes 18% longer).  Transient FP64, against the element
+// kernel with its 4.6 KB of blocks per element and the gather: 128^3 8.23 -> 2.84 ms, 96^3 3.61 ->
+// 1.21 ms, 18^3 238 -> 28 us.
 struct Elastic8GParams {
   Elastic8Params p;
   const double *X, *Y, *Z;
@@ -1393,39 +1397,60 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
   const double lamf = p.nu / ((1.0 + p.nu) * (1.0 - 2.0 * p.nu)), muf = 0.5 / (1.0 + p.nu);
   const double cK = TR ? p.beta + p.alpha * p.rb : p.beta;
   const double cM = TR ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
+  // A tile's vertices (clamped into the mesh: what lies outside belongs to no cell of the mesh) are
+  // loaded while the tile before is computed, ahead of its row stores: one counter tracks a wave's
+  // loads and stores, so loads issued after the stores would wait for them.
+  double vx[3], vu[3], vm[3];
+  auto load_vertex = [&](int tile) {
+    const int t = min(tid, kV8 - 1);
+    const int I0 = tile % gx * kN8, J0 = tile / gx % gy * kN8, K = tile / (gx * gy);
+    const int ix = min(max(I0 - 1 + t % (kN8 + 2), 0), p.nx);
+    const int iy = min(max(J0 - 1 + t / (kN8 + 2) % (kN8 + 2), 0), p.ny);
+    const int iz = min(max(K - 1 + t / ((kN8 + 2) * (kN8 + 2)), 0), p.nz);
+    const int vi = ix + sx * iy + sxy * iz;
+    const int32_t L = p.point_lid[3 * vi];
+    vx[0] = gp.X[vi];
+    vx[1] = gp.Y[vi];
+    vx[2] = gp.Z[vi];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      vu[j] = p.x[L + j];
+      if constexpr (TR) {
+        const double v = p.xdot[L + j], a = tra ? p.xddot[L + j] : 0.0;
+        vu[j] += p.rb * v;
+        vm[j] = p.ra * v + a;
+      }
+    }
+  };
+  // LID of this lane's node and modulus of its cell, with the tile's vertices
+  int32_t Ln;
+  double En;
+  auto load_node = [&](int tile) {
+    const int I = tile % gx * kN8 + n, J = tile / gx % gy * kN8 + w, K = tile / (gx * gy);
+    Ln = p.point_lid[3 * (min(I, p.nx) + sx * min(J, p.ny) + sxy * K)];
+    const int cx = min(max(I - 1 + ox, 0), p.nx - 1), cy = min(max(J - 1 + oy, 0), p.ny - 1),
+              cz = min(max(K - 1 + oz, 0), p.nz - 1);
+    En = p.coef[cx + p.nx * (cy + p.ny * cz)];
+  };
+  load_vertex(min(static_cast<int>(blockIdx.x), ntile - 1));
+  load_node(min(static_cast<int>(blockIdx.x), ntile - 1));
   for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
     asm volatile("" : "+v"(tid));   // the staging indices are formed per tile, not kept in registers
     const int I0 = tile % gx * kN8, J0 = tile / gx % gy * kN8, K = tile / (gx * gy);
-    // vertices (clamped into the mesh: what lies outside belongs to no cell of the mesh)
-    if (tid < kV8) {
-      const int vx = min(max(I0 - 1 + tid % (kN8 + 2), 0), p.nx);
-      const int vy = min(max(J0 - 1 + tid / (kN8 + 2) % (kN8 + 2), 0), p.ny);
-      const int vz = min(max(K - 1 + tid / ((kN8 + 2) * (kN8 + 2)), 0), p.nz);
-      const int vi = vx + sx * vy + sxy * vz;
-      const int32_t L = p.point_lid[3 * vi];
-      vtx[0][tid] = gp.X[vi];
-      vtx[1][tid] = gp.Y[vi];
-      vtx[2][tid] = gp.Z[vi];
+    if (tid < kV8)
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const double u = p.x[L + j];
-        if constexpr (TR) {
-          const double v = p.xdot[L + j], a = tra ? p.xddot[L + j] : 0.0;
-          vtx[3 + j][tid] = u + p.rb * v;
-          vtx[6 + j][tid] = p.ra * v + a;
-        } else {
-          vtx[3 + j][tid] = u;
-        }
+        vtx[j][tid] = vx[j];
+        vtx[3 + j][tid] = vu[j];
+        if constexpr (TR) vtx[6 + j][tid] = vm[j];
       }
-    }
-    // this lane's node and cell: their loads go out before the barrier
+    // this lane's node and cell
     const int I = I0 + n, Jy = J0 + w;
     const bool node_ok = I <= p.nx && Jy <= p.ny;
-    const int nodev = min(I, p.nx) + sx * min(Jy, p.ny) + sxy * K;
-    const int32_t L0 = p.point_lid[3 * nodev];
+    const int32_t L0 = Ln;
     const int cx = I - 1 + ox, cy = Jy - 1 + oy, cz = K - 1 + oz;
     const bool cell_ok = node_ok && cx >= 0 && cx < p.nx && cy >= 0 && cy < p.ny && cz >= 0 && cz < p.nz;
-    const double E = p.coef[cell_ok ? cx + p.nx * (cy + p.ny * cz) : 0];
+    const double E = En;
     __syncthreads();
     // points of the cells
 #pragma unroll 1
@@ -1495,6 +1520,8 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
       rr[i] = r;
     }
     if (p.f && node_ok && l16 < 3) p.f[L0 + l16] = l16 == 0 ? rr[0] : (l16 == 1 ? rr[1] : rr[2]);
+    load_vertex(min(tile + static_cast<int>(gridDim.x), ntile - 1));
+    load_node(min(tile + static_cast<int>(gridDim.x), ntile - 1));
     if (p.vals) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
@@ -1549,7 +1576,9 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
 
 // The same row blocks on an uploaded hex8 mesh (one block): one wave per two nodes (LIDs 3 n, 3 n + 1,
 // 3 n + 2), 32 lanes per node: lane (element instance c of eight at a time, corner y and z) forms the
-// blocks of the two vertices along x.  Instances come from the node's list (ascending), the row
+// blocks of the two vertices along x.  Bound by latency at two waves per SIMD (245 VGPRs, 16 KB of LDS
+// per wave) and VALU issue (about 800 instructions per node: no two nodes share a point table).
+// Transient FP64, shuffled 64x61x67: 1.19 -> 0.64 ms (element kernel and gather before).  Instances come from the node's list (ascending), the row
 // positions from their slot maps; the blocks are added into the node's rows in LDS instance by
 // instance, so the sums have a fixed order, and the rows are stored once.
 struct Elastic8UParams {
@@ -1577,12 +1606,49 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
   const double cK = TR ? p.beta + p.alpha * p.rb : p.beta;
   const double cM = TR ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
   const int64_t npair = (gp.nnodes + 1) / 2;
+  // The first eight instances of a pair are found and their coordinates loaded while the pair before
+  // is computed, a step of the chain (list ends, instance, vertices, coordinates) at a time, the
+  // coordinates ahead of that pair's row stores.
+  int64_t rn[3];            // list ends of both nodes
+  int32_t on[3];            // instance of this lane's points for either node, and of its blocks
+  int64_t vn[2];
+  int32_t Ln[2];
+  double Xn[2][3];
+  auto load_ends = [&](int64_t pair) {
+    const int64_t q = min(pair, npair - 1);
+    rn[0] = gp.occ_ptr[2 * q];
+    rn[1] = gp.occ_ptr[2 * q + 1];
+    rn[2] = gp.occ_ptr[min(2 * q + 2, gp.nnodes)];
+  };
+  // (past a list's end: its first instance, never used)
+  auto load_occ = [&]() {
+    const int64_t k = lane >> 3;
+    on[0] = gp.occ[rn[0] + k < rn[1] ? rn[0] + k : rn[0]];
+    on[1] = gp.occ[rn[1] + k < rn[2] ? rn[1] + k : rn[0]];
+    const int64_t lo = n ? rn[1] : rn[0], hi = n ? rn[2] : rn[1];
+    on[2] = gp.occ[lo + c < hi ? lo + c : rn[0]];
+  };
+  auto load_vertices = [&]() {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      vn[m] = gp.conn[(static_cast<int64_t>(on[m]) & ~int64_t(7)) + ts];
+      Ln[m] = gp.elem_lid[((static_cast<int64_t>(on[2]) & ~int64_t(7)) + ((bb | m) ^ ((bb >> 1) & 1))) * 3];
+    }
+  };
+  auto load_coords = [&]() {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) { Xn[m][0] = gp.X[vn[m]]; Xn[m][1] = gp.Y[vn[m]]; Xn[m][2] = gp.Z[vn[m]]; }
+  };
+  load_ends(blockIdx.x);
+  load_occ();
+  load_vertices();
+  load_coords();
   for (int64_t pair = blockIdx.x; pair < npair; pair += gridDim.x) {
     const int64_t node0 = 2 * pair, node = min(node0 + n, gp.nnodes - 1);
     const bool node_ok = node0 + n < gp.nnodes;
     // instance ranges of both nodes (wave-uniform) and of this lane's
-    const int64_t r0 = gp.occ_ptr[node0], r1 = gp.occ_ptr[node0 + 1];
-    const int64_t r2 = gp.occ_ptr[min(node0 + 2, gp.nnodes)];
+    const int64_t r0 = rn[0], r1 = rn[1], r2 = rn[2];
+    load_ends(pair + gridDim.x);
     const int64_t first = n ? r1 : r0;
     const int cnt = node_ok ? static_cast<int>((n ? r2 : r1) - first) : 0;
     const int most = max(static_cast<int>(r1 - r0), static_cast<int>(r2 - r1));
@@ -1592,6 +1658,7 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
     if (p.vals)
       for (int k = lane; k < 2 * kRow8; k += 64) (&rows[0][0])[k] = 0.0;
     double racc[3] = {0.0, 0.0, 0.0};
+    const int32_t on2 = on[2], L2[2] = {Ln[0], Ln[1]};
     for (int g = 0; g < most; g += 8) {
       // points: eight lanes per instance, node 0's instances, then node 1's
 #pragma unroll
@@ -1599,14 +1666,19 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
         const int64_t lo = m ? r1 : r0, hi = m ? r2 : r1;
         const int64_t k = lo + g + (lane >> 3);
         const bool ok = k < hi;
-        const int64_t e = ok ? gp.occ[k] >> 3 : 0;
-        const int64_t v = gp.conn[8 * e + ts];
-        point_entry(gp.X[v], gp.Y[v], gp.Z[v], t, ok, tab + (m * 8 + (lane >> 3)) * 8 * kPtStride);
+        double X = Xn[m][0], Y = Xn[m][1], Z = Xn[m][2];
+        if (g > 0) {   // a node of more than eight instances (uniform over the wave)
+          const int64_t v = gp.conn[(ok ? static_cast<int64_t>(gp.occ[k]) & ~int64_t(7) : 0) + ts];
+          X = gp.X[v];
+          Y = gp.Y[v];
+          Z = gp.Z[v];
+        }
+        point_entry(X, Y, Z, t, ok, tab + (m * 8 + (lane >> 3)) * 8 * kPtStride);
       }
       // this lane's instance, its modulus, vertices' state and row positions
       const bool ok = g + c < cnt;
       const int64_t k = ok ? first + g + c : r0;
-      const int32_t occ = gp.occ[k];
+      const int32_t occ = g == 0 ? on2 : gp.occ[k];
       const int64_t e = occ >> 3;
       const int as = occ & 7, av = as ^ ((as >> 1) & 1);
       const double E = p.coef[e];
@@ -1615,7 +1687,7 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         const int bs = (bb | b) ^ ((bb >> 1) & 1);
-        const int32_t L = gp.elem_lid[(8 * e + bs) * 3];
+        const int32_t L = g == 0 ? L2[b] : gp.elem_lid[(8 * e + bs) * 3];
         pos[b] = gp.slot[8 * k + bs];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -1628,9 +1700,11 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
           }
         }
       }
+      if (g == 0) load_occ();
       gather_lds_sync();
       double T[2][3][3], M[2], m0;
       row_blocks<1, TR>(tab + (n * 8 + c) * 8 * kPtStride, bb, av ^ bb, T, M, m0);
+      if (g == 0) load_vertices();
       const double lam = ok ? E * lamf : 0.0, mu = ok ? E * muf : 0.0;
       if (!ok) m0 = 0.0;
       double rr[3] = {0.0, 0.0, 0.0};
@@ -1675,6 +1749,7 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
       }
       gather_lds_sync();   // the points are read; the next eight instances go over them
     }
+    load_coords();
     // residual over the node's 32 lanes (the total ends in the second row of 16), rows
 #pragma unroll
     for (int i = 0; i < 3; ++i) racc[i] = group_sum<32>(racc[i]);
@@ -1710,14 +1785,14 @@ size_t ws_round(size_t b) { return (b + kWsAlign - 1) / kWsAlign * kWsAlign; }
 // workspace bytes: residuals [E][ND] FP64 when f is wanted, blocks [E][ND][ND] when vals are
 // affine HEX8 bricks take the node-centric kernel (no workspace) in every precision
 bool affine_hex8(const Mesh &m) {
-  return m.topo == TXA_HEX8 && m.affine && m.structured && m.nfields == 3 && m.npoints < (int64_t(1) << 31);
+  return m.topo == TXA_HEX8 && m.affine && m.structured && m.nfields == 3;
 }
 
 // hex8 elasticity on general cells in FP64: the node kernels on bricks and on uploads whose
 // rows fit them
 bool general_hex8(const Mesh &m, int precision) {
   if (m.topo != TXA_HEX8 || m.nfields != 3 || precision != TXA_FP64) return false;
-  return m.structured ? !m.affine && m.npoints < (int64_t(1) << 31) : m.uocc.p != nullptr;
+  return m.structured ? !m.affine : m.uocc.p != nullptr;   // three int32 LIDs per point: under 2^31 points
 }
 
 // Streams and events of the element / gather slab pipeline, one set per host thread and device
@@ -1744,10 +1819,6 @@ SlabPipe &slab_pipe(int dev) {
 }
 
 void ws_parts(const Mesh &m, int precision, bool want_f, bool want_vals, size_t *rbytes, size_t *jbytes) {
-  if (affine_hex8(m)) {
-    *rbytes = *jbytes = 0;
-    return;
-  }
   const size_t nd = static_cast<size_t>(m.ndof_elem), ne = static_cast<size_t>(m.nelem);
   *rbytes = want_f ? ws_round(ne * nd * sizeof(double)) : 0;
   const size_t nb = nd / 3;
@@ -1764,8 +1835,9 @@ bool elastic_supported(const Mesh &m, const txa_assembly_args &a) {
   return m.topo == TXA_HEX27;
 }
 
-size_t elastic_workspace_bytes(const Mesh &m, int precision, bool want_f, bool want_vals) {
+size_t elastic_workspace_bytes(const Mesh &m, int precision, bool want_f, bool want_vals, bool footprint) {
   size_t r = 0, j = 0;
+  if (affine_hex8(m) || (!footprint && general_hex8(m, precision))) return 0;
   ws_parts(m, precision, want_f, want_vals, &r, &j);
   return r + j;
 }
@@ -1926,8 +1998,7 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
   p.jbuf = jbytes ? static_cast<void *>(w + rbytes) : nullptr;
   auto elem_launch = [&](const ElasticParams &pp, hipStream_t st) {
     if (m.topo == TXA_HEX8) {
-      if (a.precision == TXA_FP32) launch<8, 8, 64, MODE_F32>(pp, st);
-      else launch<8, 8, 64, MODE_F64>(pp, st);
+      launch<8, 8, 64, MODE_F32>(pp, st);   // FP64: the node kernels
     } else {
       if (a.precision == TXA_SPLIT_BF16) launch<27, 27, 256, MODE_SPLIT>(pp, st);
       else if (a.precision == TXA_FP32) launch<27, 27, 256, MODE_F32>(pp, st);
@@ -1952,8 +2023,7 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
     u.vals = a.vals;
     const unsigned ug = static_cast<unsigned>(std::min<int64_t>((u.nnodes + 3) / 4, static_cast<int64_t>(ncu) * 16));
     if (m.topo == TXA_HEX8) {
-      if (wide) hipLaunchKernelGGL((k_elastic_gather_u<8, double>), dim3(ug), dim3(256), 0, s, u);
-      else hipLaunchKernelGGL((k_elastic_gather_u<8, float>), dim3(ug), dim3(256), 0, s, u);
+      hipLaunchKernelGGL((k_elastic_gather_u<8, float>), dim3(ug), dim3(256), 0, s, u);
     } else {
       if (wide) hipLaunchKernelGGL((k_elastic_gather_u<27, double>), dim3(ug), dim3(256), 0, s, u);
       else hipLaunchKernelGGL((k_elastic_gather_u<27, float>), dim3(ug), dim3(256), 0, s, u);
@@ -1979,8 +2049,7 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
   auto gather_launch = [&](const GatherParams &gg, hipStream_t st) {
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>((gg.p1 - gg.p0 + 3) / 4, static_cast<int64_t>(ncu) * 16));
     if (m.topo == TXA_HEX8) {
-      if (wide) hipLaunchKernelGGL((k_elastic_gather<8, double>), dim3(grid), dim3(256), 0, st, gg);
-      else hipLaunchKernelGGL((k_elastic_gather<8, float>), dim3(grid), dim3(256), 0, st, gg);
+      hipLaunchKernelGGL((k_elastic_gather<8, float>), dim3(grid), dim3(256), 0, st, gg);
     } else {
       if (wide) hipLaunchKernelGGL((k_elastic_gather<27, double>), dim3(grid), dim3(256), 0, st, gg);
       else hipLaunchKernelGGL((k_elastic_gather<27, float>), dim3(grid), dim3(256), 0, st, gg);

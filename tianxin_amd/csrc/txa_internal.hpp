@@ -232,8 +232,12 @@ void upload_block_refs(Mesh &m, hipStream_t s);   // tables of the mesh's topolo
 // the work on s (may be null when that size is 0)
 // err: device (or host-mapped) int set to 1 when a Dirichlet LID lies outside the map (may be null)
 void assemble(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws, int *err = nullptr);
+// Workspace an assembly uses.  footprint: the size that bounds what txa_assemble_noalloc and a server
+// accept, which counts element blocks for every elasticity call on cells that are not parallelepipeds,
+// also where the kernel does without them (what callers see refused or queued does not move with the
+// kernels).
 size_t assemble_workspace_bytes(const Mesh &m, int physics, int precision, bool want_f, bool want_vals,
-                                bool accumulate = false);
+                                bool accumulate = false, bool footprint = false);
 void apply_dirichlet(const Mesh &m, const int32_t *lids, const double *g, int64_t n, const double *x, double *f,
                      double *vals, hipStream_t s, int *err);
 void spmv(const Mesh &m, const double *vals, const double *x, double *y, hipStream_t s);
@@ -241,7 +245,7 @@ void fill_async(double *p, int64_t n, double v, hipStream_t s);
 // element-centric elasticity (txa_elastic.hip)
 void node_perm_build(Mesh &m, hipStream_t s);
 bool elastic_supported(const Mesh &m, const txa_assembly_args &a);
-size_t elastic_workspace_bytes(const Mesh &m, int precision, bool want_f, bool want_vals);
+size_t elastic_workspace_bytes(const Mesh &m, int precision, bool want_f, bool want_vals, bool footprint);
 void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws);
 // Q1 diffusion fast path and batches (txa_q1_hex8.hip)
 Q1Plan q1_plan(const Mesh &m, int ncu);

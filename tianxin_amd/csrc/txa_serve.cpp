@@ -329,7 +329,7 @@ int64_t serve_submit(Server &s, const txa_serve_request &r) {
   q->r = r;
   q->bytes_f = sizeof(double) * static_cast<size_t>(m.ndofs);
   q->bytes_v = r.want_jacobian ? sizeof(double) * static_cast<size_t>(m.nnz) : 0;
-  q->bytes_w = assemble_workspace_bytes(m, r.physics, r.precision, true, r.want_jacobian != 0);
+  q->bytes_w = assemble_workspace_bytes(m, r.physics, r.precision, true, r.want_jacobian != 0, false, true);
   TXA_REQUIRE(round_up(q->bytes_f) + round_up(q->bytes_v) + round_up(q->bytes_w) <= s.arena.cap, TXA_ERR_NOMEM,
               "request footprint exceeds the server's HBM budget");
   TXA_HIP(hipEventCreateWithFlags(&q->ev, hipEventDisableTiming));
