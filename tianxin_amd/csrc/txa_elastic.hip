@@ -1052,163 +1052,220 @@ __global__ void k_cell_geom(int nx, int ny, int nz, int64_t nv, const double *__
   g[9] = adet;
 }
 
-// Four waves per SIMD (125 VGPRs): the cell geometry is loaded with the node's second round
-// rather than a node ahead (a prefetch held 20 more registers: three waves, 3% slower).
-__global__ __launch_bounds__(256, 4) void k_elastic8_affine(Elastic8Params p) {
-  constexpr int MAXLEN = 81;   // entries per row: 27 neighbours x 3 fields
-  __shared__ double rows[4][3 * MAXLEN];
-  // the wave index is uniform: the node's lattice arithmetic runs on the scalar unit
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c = lane >> 3, b = lane & 7;
-  const int ox = c & 1, oy = (c >> 1) & 1, oz = c >> 2;   // cell (I-1+ox, J-1+oy, K-1+oz)
-  const int bxyz[3] = {b & 1, (b >> 1) & 1, b >> 2};
-  const int oxyz[3] = {ox, oy, oz};
-  // the node is vertex a = (1-ox, 1-oy, 1-oz) of cell c; vertex b lies at offset o - 1 + b
-  double S[3][3], mf = 1.0;
-  {
-    double sa[3], sb[3], fd[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      sa[d] = oxyz[d] ? -1.0 : 1.0;
-      sb[d] = bxyz[d] ? 1.0 : -1.0;
-      fd[d] = sa[d] == sb[d] ? 2.0 / 3.0 : 1.0 / 3.0;
-      mf *= fd[d];
-    }
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-      for (int n = 0; n < 3; ++n)
-        S[m][n] = m == n ? 0.5 * sa[m] * sb[m] * fd[(m + 1) % 3] * fd[(m + 2) % 3] : 0.25 * sa[m] * sb[n] * fd[3 - m - n];
+constexpr int kN8 = 4;                                      // nodes along x and y per workgroup
+constexpr int kV8 = (kN8 + 2) * (kN8 + 2) * 3;              // vertices around them
+constexpr int kC8 = (kN8 + 1) * (kN8 + 1) * 2;              // cells around them
+constexpr int kRow8 = 3 * 81;                               // entries of a node's rows at most
+
+// Lane of a node in the tile kernels: cell (ox, oy, oz) of the eight around it (I - 1 + ox, ...) and
+// half h (the vertices on the cell's low / high z side), as lane ^ = ox ^ 2 oy ^ 8 oz ^ 15 h, so that
+// the partner cell along x is lane ^ 1, along y lane ^ 2, and the (upper cell, low half) of lanes
+// 8-11 meets the (lower cell, high half) of lanes 12-15 at lane ^ 7: one DPP move each.
+struct NodeLane {
+  int ox, oy, oz, h;
+  __device__ __forceinline__ explicit NodeLane(int l16) {
+    h = (l16 >> 2) & 1;
+    const int lu = h ? l16 ^ 15 : l16;
+    ox = lu & 1;
+    oy = (lu >> 1) & 1;
+    oz = lu >> 3;
   }
-  const int dx = ox - 1 + bxyz[0], dy = oy - 1 + bxyz[1], dz = oz - 1 + bxyz[2];
-  const int slot = (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1);   // neighbour slot of vertex b
-  // 32-bit lattice arithmetic (the host takes this kernel only below 2^31 nodes)
-  const int sx = p.nx + 1, sxy = sx * (p.ny + 1), np = static_cast<int>(p.npoints);
-  const bool tr = p.transient && p.xdot;
-  const bool tra = tr && p.xddot;
-  const double lamf = p.nu / ((1.0 + p.nu) * (1.0 - 2.0 * p.nu)), muf = 0.5 / (1.0 + p.nu);
-  const double cK = tr ? p.beta + p.alpha * p.rb : p.beta;
-  const double cM = tr ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
+};
+
+// Entry of block k (vertex on the cell's outer side along x / y, or with bit 0 / 1 of k the node's own
+// side) summed over the cells that share its vertex: along x, then y, then z.
+template <int K>
+__device__ __forceinline__ double meet(double v, bool upper) {   // upper: lanes 8-15 of the node
+  if (K & 1) v += dpp_f64<0xB1, 0xf>(v);
+  if (K & 2) v += dpp_f64<0x4E, 0xf>(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x141, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x141, 0xf, 0xf, true);
+  return v + __hiloint2double(upper ? hi : 0, upper ? lo : 0);
+}
+// whether this lane writes block k's sum
+__device__ __forceinline__ bool owns_block(const NodeLane &q, int k) {
+  return (q.oz == q.h || q.h) && !((k & 1) && q.ox) && !((k & 2) && q.oy);
+}
+
+// One wave stores the rows of its line of four nodes (rows + n kRow8 in LDS, or one range where the
+// nodes' LIDs follow each other: run).
+__device__ __forceinline__ void store_line(const double *rows, double *vals, int64_t base, int len, bool run, int nok,
+                                           int lane) {
+  if (run) {
+    const int64_t base0 = __shfl(base, 0);
+    const int last = 16 * (nok - 1);
+    row_store(rows, vals + base0, static_cast<int>(__shfl(base, last) - base0) + 3 * __shfl(len, last), lane);
+  } else {
+    for (int m = 0; m < nok; ++m)
+      row_store(rows + m * kRow8, vals + __shfl(base, 16 * m), 3 * __shfl(len, 16 * m), lane);
+  }
+}
+
+// One wave per line of four nodes along x, 16 lanes per node; each lane forms the blocks of its cell's four vertices on one z side one after another.  With the
+// cell's cofactor columns signed by the node's corner (c_m s_a^m), T_ab = sum_mn c_m F_mn sigma_n c_n^T
+// where sigma_n = +1 / -1 and f_n = 2/3 / 1/3 as a and b agree or not along n, F_mm = f_d1 f_d2 / 2,
+// F_mn = f_d / 4 (d the third axis): x and y known per block, z per lane.  The state of the 6 x 3 x 3
+// vertices is staged in LDS, the next line's loaded before this line's row stores (one counter tracks
+// a wave's loads and stores); the waves of a workgroup share nothing.
+//
+// Bound by VALU issue (297 instructions per node, 73% busy at three waves per SIMD) and the row
+// stores.  Transient FP64, against one wave per node with 64 lanes of one block each, eight ordered
+// LDS adds per entry and the state loaded once per lane (390 instructions per node): 128^3 2.56 ->
+// 1.71 ms, 115^3 1.82 -> 1.22 ms, 64^3 319 -> 229 us; the same tiles staged per workgroup behind two
+// barriers at two waves per SIMD 2.15 ms at 128^3.
+template <bool TR>
+__global__ __launch_bounds__(256, 3) void k_elastic8_affine(Elastic8Params p) {
+  constexpr int NV = (kN8 + 2) * 9;
+  __shared__ double state[4][TR ? 6 : 3][NV];           // u + b_R v, a_R v + a
+  __shared__ double row[4][kN8 * kRow8];
+  int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto &vtx = state[w];
+  const int l16 = lane & 15, n = lane >> 4;
+  NodeLane q(l16);
+  const int sx = p.nx + 1, sxy = sx * (p.ny + 1);
+  const int gx = (sx + kN8 - 1) / kN8, gy = p.ny + 1;
+  const int ntile = gx * gy * (p.nz + 1);
+  const bool tra = TR && p.xddot;
+  const double ratio = 2.0 * p.nu / (1.0 - 2.0 * p.nu), muf = 0.5 / (1.0 + p.nu);
+  const double cK = TR ? p.beta + p.alpha * p.rb : p.beta;
+  const double cM = TR ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
+  double vu[3], vm[3], En;
+  int32_t Ln;
+  auto load_tile = [&](int tile) {
+    const int I0 = tile % gx * kN8, J0 = tile / gx % gy, K = tile / (gx * gy);
+    const int t = min(lane, NV - 1);
+    const int ix = min(max(I0 - 1 + t % (kN8 + 2), 0), p.nx);
+    const int iy = min(max(J0 - 1 + t / (kN8 + 2) % 3, 0), p.ny);
+    const int iz = min(max(K - 1 + t / (3 * (kN8 + 2)), 0), p.nz);
+    const int32_t L = p.point_lid[3 * (ix + sx * iy + sxy * iz)];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      vu[j] = p.x[L + j];
+      if constexpr (TR) {
+        const double v = p.xdot[L + j], a = tra ? p.xddot[L + j] : 0.0;
+        vu[j] += p.rb * v;
+        vm[j] = p.ra * v + a;
+      }
+    }
+    Ln = p.point_lid[3 * (min(I0 + n, p.nx) + sx * J0 + sxy * K)];
+    const int cx = min(max(I0 + n - 1 + q.ox, 0), p.nx - 1), cy = min(max(J0 - 1 + q.oy, 0), p.ny - 1),
+              cz = min(max(K - 1 + q.oz, 0), p.nz - 1);
+    En = p.coef[cx + p.nx * (cy + p.ny * cz)];
+  };
   const int stride = static_cast<int>(gridDim.x) * 4;
-  // Loads come in two rounds per node (the lane's vertex LID and the node's LID; then the
-  // state by that LID, the node's row pointers and slot map, and the cell's geometry and
-  // modulus).  The first round of the next node is issued before this node's arithmetic,
-  // the second round of this node as its iteration starts.
-  struct Round1 {
-    int I, J, K;
-    int32_t Lb, L0;
-  };
-  auto round1 = [&](int q, Round1 &r) {
-    const int qc = q < np ? q : np - 1;   // past the end: loaded, never used
-    r.I = qc % sx;
-    r.J = (qc / sx) % (p.ny + 1);
-    r.K = qc / sxy;
-    // this lane's vertex (clamped into the mesh for absent cells: loaded, never used)
-    const int vx = min(max(r.I + dx, 0), p.nx), vy = min(max(r.J + dy, 0), p.ny), vz = min(max(r.K + dz, 0), p.nz);
-    const int vi = vx + sx * vy + sxy * vz;
-    r.Lb = p.point_lid[3 * vi];
-    r.L0 = p.point_lid[3 * qc];
-  };
-  int pt = static_cast<int>(blockIdx.x) * 4 + w;
-  Round1 cur, nxt;
-  round1(pt, cur);
-  for (; pt < np; pt += stride) {
-    const int I = cur.I, Jy = cur.J, K = cur.K;
-    const int cx = I - 1 + ox, cy = Jy - 1 + oy, cz = K - 1 + oz;
-    const bool cell_ok = cx >= 0 && cx < p.nx && cy >= 0 && cy < p.ny && cz >= 0 && cz < p.nz;
-    // second round of this node
-    double ub[3], vb[3], ab[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      ub[j] = p.x[cur.Lb + j];
-      vb[j] = tr ? p.xdot[cur.Lb + j] : 0.0;
-      ab[j] = tra ? p.xddot[cur.Lb + j] : 0.0;
-    }
-    const int32_t L0 = cur.L0;
-    const int64_t base = p.rowptr[L0];
-    const int len = min(static_cast<int>(p.rowptr[L0 + 1] - base), MAXLEN);
-    const int node = L0 / 3;
-    const uint16_t pos = p.nperm[static_cast<int64_t>(node) * p.nperm_w + slot];
-    const int cell = cell_ok ? cx + p.nx * (cy + p.ny * cz) : 0;
-    const double E = p.coef[cell];
-    double2 G[5];
-    const double2 *gp = reinterpret_cast<const double2 *>(p.geom + 10 * static_cast<int64_t>(cell));
-#pragma unroll
-    for (int t = 0; t < 5; ++t) G[t] = gp[t];
-    // first round of the next node
-    round1(pt + stride, nxt);
-    __builtin_amdgcn_sched_barrier(0);
-    // T = C S C^T / |det J| = Chat S Chat^T with the cell's scaled cofactors
-    const double Ch[3][3] = {{G[0].x, G[0].y, G[1].x}, {G[1].y, G[2].x, G[2].y}, {G[3].x, G[3].y, G[4].x}};
-    const double adet = G[4].y;
-    double P[3][3];
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-      for (int l = 0; l < 3; ++l) P[m][l] = S[m][0] * Ch[l][0] + S[m][1] * Ch[l][1] + S[m][2] * Ch[l][2];
-    double T[3][3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int l = 0; l < 3; ++l) T[k][l] = Ch[k][0] * P[0][l] + Ch[k][1] * P[1][l] + Ch[k][2] * P[2][l];
-    const double lam = E * lamf, mu = E * muf;
-    const double trs = T[0][0] + T[1][1] + T[2][2];
-    const double Mab = tr ? p.rho * adet * mf : 0.0;
-    double rr[3] = {0.0, 0.0, 0.0};
-    double jb[9];
-    // with C = a_R M + b_R K:  J = (beta + alpha b_R) K + (alpha a_R + gamma2) M  and
-    // R = K (u + b_R v) + M (a_R v + a)
-    double ut[3], mt[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      ut[j] = tr ? ub[j] + p.rb * vb[j] : ub[j];
-      mt[j] = tr ? p.ra * vb[j] + (tra ? ab[j] : 0.0) : 0.0;
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
+  int tile = static_cast<int>(blockIdx.x) * 4 + w;
+  load_tile(min(tile, ntile - 1));
+  for (; tile < ntile; tile += stride) {
+    // indices and lane factors are formed per tile, not kept in registers
+    asm volatile("" : "+v"(lane), "+v"(q.ox), "+v"(q.oy), "+v"(q.oz), "+v"(q.h));
+    const bool zsame = q.h != q.oz;                       // b on the node's side along z
+    const double fz = zsame ? 2.0 / 3.0 : 1.0 / 3.0;
+    const int I0 = tile % gx * kN8, J0 = tile / gx % gy, K = tile / (gx * gy);
+    if (lane < NV)
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const double Kv = lam * T[i][j] + mu * T[j][i] + (i == j ? mu * trs : 0.0);
-        rr[i] += Kv * ut[j];
-        double jv = cK * Kv;
-        if (i == j) {
-          jv += cM * Mab;
-          rr[i] += Mab * mt[j];
-        }
-        jb[3 * i + j] = jv;
+        vtx[j][lane] = vu[j];
+        if constexpr (TR) vtx[3 + j][lane] = vm[j];
       }
-    // the cell's source load enters once (vertex b = a), F_a = src |det J|
-    const bool ba = b == (1 - ox) + 2 * (1 - oy) + 4 * (1 - oz);
+    const int I = I0 + n, Jy = J0;
+    const bool node_ok = I <= p.nx;
+    const int32_t L0 = Ln;
+    const int cx = I - 1 + q.ox, cy = Jy - 1 + q.oy, cz = K - 1 + q.oz;
+    const bool cell_ok = node_ok && cx >= 0 && cx < p.nx && cy >= 0 && cy < p.ny && cz >= 0 && cz < p.nz;
+    const double E = cell_ok ? En : 0.0;
+    double2 G[5];
+    const double2 *gp = reinterpret_cast<const double2 *>(p.geom + 10 * static_cast<int64_t>(cell_ok ? cx + p.nx * (cy + p.ny * cz) : 0));
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      // fixed-order sum over the wave: each half's total (DPP) ends in lanes 16 and 48
-      const double v = group_sum<32>(cell_ok ? rr[i] - (ba ? p.src[i] * adet : 0.0) : 0.0);
-      const double h0 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 16),
-                                         __builtin_amdgcn_readlane(__double2loint(v), 16));
-      const double h1 = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 48),
-                                         __builtin_amdgcn_readlane(__double2loint(v), 48));
-      rr[i] = h0 + h1;
-    }
-    // rows: zero, then the cells' blocks in cell order (every column of the rows is a neighbour
-    // within one cell, so every entry is reached)
-    for (int k = lane; k < 3 * len; k += 64) rows[w][k] = 0.0;
-    const bool add = cell_ok && pos != 0xffffu && pos + 2 < len;
+    for (int t = 0; t < 5; ++t) G[t] = gp[t];
+    const int64_t base = p.rowptr[L0];
+    const int len = min(static_cast<int>(p.rowptr[L0 + 1] - base), 81);
+    const uint16_t *np = p.nperm + static_cast<int64_t>(L0 / 3) * p.nperm_w;
+    int pos[4];
 #pragma unroll
-    for (int cc = 0; cc < 8; ++cc)
-      if (c == cc && add)
+    for (int k = 0; k < 4; ++k) pos[k] = np[((k & 1) ? 1 : 2 * q.ox) + 3 * ((k & 2) ? 1 : 2 * q.oy) + 9 * (q.oz + q.h)];
+    gather_lds_sync();
+    // cofactor columns (scaled by |det J|^-1/2), signed by the node's corner of the cell
+    const double ax = q.ox ? -1.0 : 1.0, ay = q.oy ? -1.0 : 1.0, az = q.oz ? -1.0 : 1.0;
+    const double c[3][3] = {{ax * G[0].x, ax * G[1].y, ax * G[3].x}, {ay * G[0].y, ay * G[2].x, ay * G[3].y},
+                            {az * G[1].x, az * G[2].y, az * G[4].x}};   // c[m]: column m
+    const double adet = cell_ok ? G[4].y : 0.0;
+    // the second factor carries mu: T below is mu T_ab, and lambda = mu * 2 nu / (1 - 2 nu)
+    const double mu = E * muf;
+    double cm[3][3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int l = 0; l < 3; ++l) cm[m][l] = mu * (m == 2 && !zsame ? -c[m][l] : c[m][l]);
+    const int64_t base0 = __shfl(base, 0);
+    const bool run = __all(!node_ok || L0 == __shfl(L0, 0) + 3 * n);
+    double *mine = row[w] + (run ? static_cast<int>(base - base0) : n * kRow8);
+    double rr[3] = {0.0, 0.0, 0.0};
+    auto block = [&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      constexpr double fx = (k & 1) ? 2.0 / 3.0 : 1.0 / 3.0, fy = (k & 2) ? 2.0 / 3.0 : 1.0 / 3.0;
+      constexpr double gx_ = (k & 1) ? 1.0 : -1.0, gy_ = (k & 2) ? 1.0 : -1.0;   // sigma
+      double P[3][3], T[3][3];
+#pragma unroll
+      for (int l = 0; l < 3; ++l) {
+        P[0][l] = (0.5 * fy * gx_ * fz) * cm[0][l] + (0.25 * gy_ * fz) * cm[1][l] + (0.25 * fy) * cm[2][l];
+        P[1][l] = (0.25 * gx_ * fz) * cm[0][l] + (0.5 * fx * gy_ * fz) * cm[1][l] + (0.25 * fx) * cm[2][l];
+        P[2][l] = (0.25 * fy * gx_) * cm[0][l] + (0.25 * fx * gy_) * cm[1][l] + (0.5 * fx * fy) * cm[2][l];
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int l = 0; l < 3; ++l) T[i][l] = c[0][i] * P[0][l] + c[1][i] * P[1][l] + c[2][i] * P[2][l];
+      const int bx = q.ox ^ (k & 1), by = q.oy ^ (k >> 1);
+      const int vi = (n + q.ox + bx) + (kN8 + 2) * ((q.oy + by) + 3 * (q.oz + q.h));
+      const double trs = T[0][0] + T[1][1] + T[2][2];
+      const double Mab = TR ? p.rho * adet * (fx * fy * fz) : 0.0;
+      double ut[3], mt[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) { ut[j] = vtx[j][vi]; mt[j] = TR ? vtx[TR ? 3 + j : 0][vi] : 0.0; }
+      const bool put = p.vals && node_ok && owns_block(q, k) && pos[k] + 2 < len;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const double Kv = ratio * T[i][j] + T[j][i] + (i == j ? trs : 0.0);
+          rr[i] += Kv * ut[j];
+          double jv = cK * Kv;
+          if (TR && i == j) {
+            jv += cM * Mab;
+            rr[i] += Mab * mt[j];
+          }
+          P[i][j] = meet<k>(jv, l16 > 7);
+        }
+      if (put)
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
-          for (int j = 0; j < 3; ++j) atomicAdd(&rows[w][i * len + pos + j], jb[3 * i + j]);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (p.vals) row_store(rows[w], p.vals + base, 3 * len, lane);
-    if (p.f && lane < 3) p.f[L0 + lane] = rr[lane];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    cur = nxt;
+          for (int j = 0; j < 3; ++j) mine[i * len + pos[k] + j] = P[i][j];
+      // one block's values in registers at a time: the next one's inputs wait for these sums
+      asm volatile("" : "+v"(rr[0]), "+v"(rr[1]), "+v"(rr[2]), "+v"(cm[0][0]), "+v"(cm[0][1]), "+v"(cm[0][2]),
+                   "+v"(cm[1][0]), "+v"(cm[1][1]), "+v"(cm[1][2]), "+v"(cm[2][0]), "+v"(cm[2][1]), "+v"(cm[2][2])
+                   : : "memory");
+    };
+    block(std::integral_constant<int, 0>());
+    block(std::integral_constant<int, 1>());
+    block(std::integral_constant<int, 2>());
+    block(std::integral_constant<int, 3>());
+    load_tile(min(tile + stride, ntile - 1));
+    // residual: the cell's source load enters once, then the sum over the node's 16 lanes
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      double r = rr[i] - (q.h == 0 ? p.src[i] * adet : 0.0);
+      r += dpp_f64<0xB1, 0xf>(r);
+      r += dpp_f64<0x4E, 0xf>(r);
+      r += dpp_f64<0x141, 0xf>(r);
+      r += dpp_f64<0x140, 0xf>(r);
+      rr[i] = r;
+    }
+    if (p.f && node_ok && l16 < 3) p.f[L0 + l16] = l16 == 0 ? rr[0] : (l16 == 1 ? rr[1] : rr[2]);
+    gather_lds_sync();   // a wave writes and reads its own line's rows
+    if (p.vals) store_line(row[w], p.vals, base, len, run, min(kN8, sx - I0), lane);
+    gather_lds_sync();   // the staged state and the rows are read
   }
 }
 
@@ -1372,11 +1429,6 @@ struct Elastic8GParams {
   const double *X, *Y, *Z;
 };
 
-constexpr int kN8 = 4;                                      // nodes along x and y per workgroup
-constexpr int kV8 = (kN8 + 2) * (kN8 + 2) * 3;              // staged vertices
-constexpr int kC8 = (kN8 + 1) * (kN8 + 1) * 2;              // cells
-constexpr int kRow8 = 3 * 81;                               // entries of a node's rows at most
-
 template <bool TR>
 __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp) {
   const Elastic8Params &p = gp.p;
@@ -1385,11 +1437,9 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
   static_assert(kN8 * kN8 * kRow8 <= kC8 * 8 * kPtStride, "rows fit over the point table");
   int tid = threadIdx.x;
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // lane of a node = ox ^ 2 oy ^ 8 oz ^ 15 h: the partner cell along x is lane ^ 1, along y lane ^ 2,
-  // and the (upper cell, low half) of lanes 8-11 meets the (lower cell, high half) of lanes 12-15
-  // at lane ^ 7: one DPP move each
-  const int l16 = lane & 15, lu = (l16 & 4) ? l16 ^ 15 : l16;
-  const int n = lane >> 4, h = (l16 >> 2) & 1, ox = lu & 1, oy = (lu >> 1) & 1, oz = lu >> 3;
+  const int l16 = lane & 15, n = lane >> 4;
+  const NodeLane q(l16);
+  const int ox = q.ox, oy = q.oy, oz = q.oz, h = q.h;
   const int sx = p.nx + 1, sxy = sx * (p.ny + 1);
   const int gx = (sx + kN8 - 1) / kN8, gy = (p.ny + 1 + kN8 - 1) / kN8;
   const int ntile = gx * gy * (p.nz + 1);
@@ -1524,18 +1574,14 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
     load_node(min(tile + static_cast<int>(gridDim.x), ntile - 1));
     if (p.vals) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            double v = T[k][i][j];
-            if (k & 1) v += dpp_f64<0xB1, 0xf>(v);   // the cells on both sides along x
-            if (k & 2) v += dpp_f64<0x4E, 0xf>(v);   // along y
-            const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x141, 0xf, 0xc, false);
-            const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x141, 0xf, 0xc, false);
-            T[k][i][j] = v + __hiloint2double(hi, lo);   // along z (lanes 8-15)
-          }
+        for (int j = 0; j < 3; ++j) {
+          T[0][i][j] = meet<0>(T[0][i][j], l16 > 7);
+          T[1][i][j] = meet<1>(T[1][i][j], l16 > 7);
+          T[2][i][j] = meet<2>(T[2][i][j], l16 > 7);
+          T[3][i][j] = meet<3>(T[3][i][j], l16 > 7);
+        }
     }
     __syncthreads();   // every wave is done with the points and the vertices: the rows go over the points
     if (p.vals) {
@@ -1545,10 +1591,9 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
       const bool run = __all(!node_ok || L0 == L00 + 3 * n);
       double *rows = tab + w * kN8 * kRow8;
       double *mine = rows + (run ? static_cast<int>(base - base0) : n * kRow8);
-      const bool zown = (oz == h) || h;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        if (node_ok && pos[k] + 2 < len && zown && !((k & 1) && ox) && !((k & 2) && oy)) {
+        if (node_ok && pos[k] + 2 < len && owns_block(q, k)) {
 #pragma unroll
           for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -1556,19 +1601,7 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
         }
       }
       gather_lds_sync();
-      const int nok = min(kN8, sx - I0);   // nodes of the line inside the mesh
-      if (Jy <= p.ny) {
-        if (run) {
-          const int last = 16 * (nok - 1);
-          const int total = static_cast<int>(__shfl(base, last) - base0) + 3 * __shfl(len, last);
-          row_store(rows, p.vals + base0, total, lane);
-        } else {
-          for (int m = 0; m < nok; ++m) {
-            const int64_t bm = __shfl(base, 16 * m);
-            row_store(rows + m * kRow8, p.vals + bm, 3 * __shfl(len, 16 * m), lane);
-          }
-        }
-      }
+      if (Jy <= p.ny) store_line(rows, p.vals, base, len, run, min(kN8, sx - I0), lane);
     }
     __syncthreads();
   }
@@ -1925,6 +1958,11 @@ Elastic8Params elastic8_params(const Mesh &m, const txa_assembly_args &a) {
   return q;
 }
 
+// tiles of the hex8 node kernels on a brick
+int64_t tiles8(const Mesh &m) {
+  return static_cast<int64_t>((m.nx + kN8) / kN8) * ((m.ny + kN8) / kN8) * (m.nz + 1);
+}
+
 // workgroups for a grid-stride kernel: the resident ones, or as many as there are items
 template <class Kernel>
 unsigned resident_grid(Kernel k, int64_t items, int threads = 256) {
@@ -1943,7 +1981,11 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
   if (affine_hex8(m)) {
     TXA_REQUIRE(m.cell_geom.p != nullptr, TXA_ERR_LOGIC, "cell geometry missing (graph_build)");
     const Elastic8Params q = elastic8_params(m, a);
-    hipLaunchKernelGGL(k_elastic8_affine, dim3(resident_grid(k_elastic8_affine, (m.npoints + 3) / 4)), dim3(256), 0, s, q);
+    const int64_t groups = (static_cast<int64_t>((m.nx + kN8) / kN8) * (m.ny + 1) * (m.nz + 1) + 3) / 4;   // four lines each
+    if (a.transient && a.xdot)
+      hipLaunchKernelGGL(k_elastic8_affine<true>, dim3(resident_grid(k_elastic8_affine<true>, groups)), dim3(256), 0, s, q);
+    else
+      hipLaunchKernelGGL(k_elastic8_affine<false>, dim3(resident_grid(k_elastic8_affine<false>, groups)), dim3(256), 0, s, q);
     TXA_HIP(hipGetLastError());
     return;
   }
@@ -1951,7 +1993,7 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
     Elastic8GParams q;
     q.p = elastic8_params(m, a);
     q.X = m.xyz.p; q.Y = m.xyz.p + m.nverts; q.Z = m.xyz.p + 2 * m.nverts;
-    const int64_t tiles = static_cast<int64_t>((m.nx + 1 + kN8 - 1) / kN8) * ((m.ny + 1 + kN8 - 1) / kN8) * (m.nz + 1);
+    const int64_t tiles = tiles8(m);
     if (a.transient && a.xdot)
       hipLaunchKernelGGL(k_elastic8_general<true>, dim3(resident_grid(k_elastic8_general<true>, tiles)), dim3(256), 0, s, q);
     else
