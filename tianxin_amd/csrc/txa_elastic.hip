@@ -1796,6 +1796,394 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
   }
 }
 
+// hex27 bricks, FP64 calls that want the matrix: node rows without element blocks.  k_points27 writes the
+// points of each cell (27 x 128 bytes); one wave then owns the nodes of a line along x of one class, the
+// parity (py, pz) of their y and z lattice coordinates, and marches over the line's cells.  The cells
+// around such a line are 4, 2, 2 or 1 per x position for (py, pz) = (0,0), (1,0), (0,1), (1,1).  Per cell
+// the wave forms the 3 x 3 blocks of its three nodes (x lattice 0, 1, 2 of the cell) with the cell's 27
+// nodes on v_mfma_f64_16x16x4f64:
+//   T[(a,k),(b,l)] = sum_q s_q (C dN_a)_k (C dN_b)_l,   C the cofactors of J, s = w / det.
+// Operand row l % 16 = a + 4 k, columns b in two tiles per l: as lane l of the product holds D rows
+// l / 16 + 4 i, it ends up with all nine entries of the pair (a = l / 16, b = l % 16), so no Gram matrix
+// goes through LDS.  Row group 3 is w det N_a: with columns N_b it gives the mass matrix, and its sum over
+// the points the source load.  A lane holds one of the 16 values of each of its row's points (one coalesced
+// load per cell) and the operands are formed from DPP broadcasts of them and the wave's constant dN_b:
+// read from LDS instead (16 lanes the same 16 bytes), they took 61% of its cycles (1.84 ms against 1.53 at
+// 33^3).  Blocks are added in lattice order into the rows in LDS (one wave's LDS operations execute in order
+// and the lanes of one add hit distinct entries: a fixed order of sums, the same for every split of a
+// line), and rows are stored once in CRS order when their last cell is done.
+//
+// Bound by issue: of 2.6 M cycles per SIMD at 33^3 the products take 0.9 M (46% of their rows and columns
+// are used) and 218 k VALU instructions 0.87 M, at seven waves per CU (22.8 KB of LDS, 256 VGPRs).  Steady
+// FP64 33^3, against the element kernel with its 55 KB of blocks per element and the gather: 1.79 -> 1.17 ms.
+// The FP32 and split-BF16 forms keep those: their results are rounded there.
+struct Node27Params {
+  Elastic8Params p;
+  const double *pts;        // [cells][27][4][4]: rows k of C with s; w det, 0, 0, 1
+  int chunk, nchunk;        // x positions per workgroup, workgroups per line
+};
+
+__global__ __launch_bounds__(256) void k_points27(int nx, int ny, int64_t ncell, const double *__restrict__ X,
+                                                  const double *__restrict__ Y, const double *__restrict__ Z,
+                                                  double *__restrict__ pts) {
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (id >= ncell * 27) return;
+  const int64_t c = id / 27;
+  const int q = static_cast<int>(id - 27 * c), qd[3] = {q % 3, q / 3 % 3, q / 9};
+  const int64_t i = c % nx, j = c / nx % ny, k = c / (static_cast<int64_t>(nx) * ny);
+  const int64_t v0 = i + (nx + 1) * (j + static_cast<int64_t>(ny + 1) * k), sy = nx + 1,
+                sz = static_cast<int64_t>(nx + 1) * (ny + 1);
+  double L[2][3], w = 1.0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const double xi = (qd[d] - 1) * 0.77459666924148337704;
+    L[0][d] = 0.5 * (1.0 - xi);
+    L[1][d] = 0.5 * (1.0 + xi);
+    w *= qd[d] == 1 ? 8.0 / 9.0 : 5.0 / 9.0;
+  }
+  double J[3][3] = {};
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int ox = kHexV[b][0], oy = kHexV[b][1], oz = kHexV[b][2];
+    const int64_t v = v0 + ox + oy * sy + oz * sz;
+    const double gx = L[ox][0], gy = L[oy][1], gz = L[oz][2], P[3] = {X[v], Y[v], Z[v]};
+    const double d[3] = {(ox ? 0.5 : -0.5) * gy * gz, gx * (oy ? 0.5 : -0.5) * gz, gx * gy * (oz ? 0.5 : -0.5)};
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) J[i][j] += P[i] * d[j];
+  }
+  double C[9];
+  C[0] = J[1][1] * J[2][2] - J[1][2] * J[2][1];
+  C[1] = J[1][2] * J[2][0] - J[1][0] * J[2][2];
+  C[2] = J[1][0] * J[2][1] - J[1][1] * J[2][0];
+  C[3] = J[0][2] * J[2][1] - J[0][1] * J[2][2];
+  C[4] = J[0][0] * J[2][2] - J[0][2] * J[2][0];
+  C[5] = J[0][1] * J[2][0] - J[0][0] * J[2][1];
+  C[6] = J[0][1] * J[1][2] - J[0][2] * J[1][1];
+  C[7] = J[0][2] * J[1][0] - J[0][0] * J[1][2];
+  C[8] = J[0][0] * J[1][1] - J[0][1] * J[1][0];
+  const double det = J[0][0] * C[0] + J[0][1] * C[1] + J[0][2] * C[2];
+  const double s = w / det;
+  double2 *o = reinterpret_cast<double2 *>(pts + 16 * id);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    o[2 * k] = make_double2(C[3 * k], C[3 * k + 1]);
+    o[2 * k + 1] = make_double2(C[3 * k + 2], s);
+  }
+  o[6] = make_double2(w * det, 0.0);
+  o[7] = make_double2(0.0, 1.0);
+}
+
+constexpr int rows27(int n9) { return 5 * n9 + 2 * 3 * n9; }   // current, middle and next nodes of a line
+constexpr int kRows27 = rows27(25 * 9);
+
+// entry N of the row of 16 lanes' values, in all its lanes; entry N of each quad's
+template <int N>
+__device__ __forceinline__ double row_entry(double v) { return __builtin_amdgcn_update_dpp(v, v, 0x150 + N, 0xf, 0xf, true); }
+template <int N>
+__device__ __forceinline__ double quad_entry(double v) {
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), N * 0x55, 0xf, 0xf, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), N * 0x55, 0xf, 0xf, true));
+}
+
+// Stores a node's three rows from lattice order (slot (dx Dy + dy) Dz + dz, nine entries each) in CRS
+// order.  np0, np1: the node's nperm entries lane, lane + 64; inv: of each neighbour, its slot's entries.
+__device__ __forceinline__ void store_node27(const double *buf, uint16_t *inv, int rx, int ry, int rz, int np0, int np1,
+                                             double *vals, int64_t base, int len, int lane) {
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int s = lane + 64 * r, ps = r ? np1 : np0;
+    const int dx = s % 5 - 2 + rx, dy = s / 5 % 5 - 2 + ry, dz = s / 25 - 2 + rz;
+    if (s < 125 && ps < 375) inv[ps / 3] = static_cast<uint16_t>(9 * ((dx * (2 * ry + 1) + dy) * (2 * rz + 1) + dz));
+  }
+  gather_lds_sync();
+  double *dst = vals + base;
+#pragma unroll 1
+  for (int k = lane; k < len; k += 64) {
+    const int nb = (k * 21846) >> 16;   // k / 3
+    const double *b = buf + inv[nb] + (k - 3 * nb);
+    __builtin_nontemporal_store(b[0], dst + k);
+    __builtin_nontemporal_store(b[3], dst + len + k);
+    __builtin_nontemporal_store(b[6], dst + 2 * len + k);
+  }
+}
+
+template <bool TR>
+__global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
+  const Elastic8Params &p = gp.p;
+  __shared__ double mem[kRows27];
+  __shared__ double2 T1[9];          // 1D basis: value and derivative of node d at Gauss point q, [3 d + q]
+  __shared__ double TA[9][3][9];     // [node y + 3 z][N N', N' N, N N of y, z][point y + 3 z]: of the row operand
+  __shared__ uint16_t inv[128];
+  __shared__ double st[27][TR ? 6 : 3];   // the cell's nodes: u + b_R v, a_R v + a
+  const int lane = threadIdx.x;
+  if (threadIdx.x < 9) {
+    const int d = threadIdx.x / 3;
+    const double xi = (static_cast<int>(threadIdx.x) % 3 - 1) * 0.77459666924148337704;
+    T1[threadIdx.x] = d == 0 ? make_double2(0.5 * xi * (xi - 1.0), xi - 0.5)
+                             : (d == 1 ? make_double2(1.0 - xi * xi, -2.0 * xi) : make_double2(0.5 * xi * (xi + 1.0), xi + 0.5));
+  }
+  __syncthreads();
+  for (int i = lane; i < 81; i += 64) {
+    const int n = i / 9, q = i % 9;
+    const double2 y = T1[3 * (n % 3) + q % 3], z = T1[3 * (n / 3) + q / 3];
+    TA[n][0][q] = y.x * z.x;
+    TA[n][1][q] = y.y * z.x;
+    TA[n][2][q] = y.x * z.y;
+  }
+  __syncthreads();
+  const int px = 2 * p.nx + 1, py = 2 * p.ny + 1;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int ka = l16 >> 2, ax = min(l16 & 3, 2);   // operand row: node ax, component ka (3: the mass row)
+  // nodes of this lane's columns, their lattice offsets and constant gradients at the points 4 ks + g
+  int bo[2][3];
+  double dB[2][7][3];
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb) {
+    const int b = min(16 * cb + l16, 26);   // any order of the 27 nodes: x fastest
+    bo[cb][0] = b % 3;
+    bo[cb][1] = b / 3 % 3;
+    bo[cb][2] = b / 9;
+#pragma unroll
+    for (int ks = 0; ks < 7; ++ks) {
+      const int q = min(4 * ks + g, 26);
+      const double2 x = T1[3 * bo[cb][0] + q % 3], y = T1[3 * bo[cb][1] + q / 3 % 3], z = T1[3 * bo[cb][2] + q / 9];
+      dB[cb][ks][0] = x.y * y.x * z.x;
+      dB[cb][ks][1] = x.x * y.y * z.x;
+      dB[cb][ks][2] = x.x * y.x * z.y;
+#pragma unroll
+      for (int m = 0; m < 3; ++m) asm volatile("" : "+v"(dB[cb][ks][m]));
+    }
+  }
+  // node min(lane, 26)'s LID entry from the cell's first
+  const int bl = min(lane, 26);
+  const unsigned lo = 3 * (bl % 3 + px * (bl / 3 % 3 + py * (bl / 9)));
+  // the row node's x basis at point 4 ks + g, of index (ks + g) % 3 along x: entry ks % 3
+  double xa[3], xd[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const double2 t = T1[3 * ax + (r + g) % 3];
+    xa[r] = t.x;
+    xd[r] = t.y;
+    if (ka == 3) xd[r] = t.x;   // the mass row takes N_a alone
+    asm volatile("" : "+v"(xa[r]), "+v"(xd[r]));
+  }
+  const bool tra = TR && p.xddot;
+  const double lamf = p.nu / ((1.0 + p.nu) * (1.0 - 2.0 * p.nu)), muf = 0.5 / (1.0 + p.nu);
+  const double cK = TR ? p.beta + p.alpha * p.rb : p.beta;
+  const double cM = TR ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
+  using cint = const __attribute__((address_space(4))) int32_t;
+  using clong = const __attribute__((address_space(4))) int64_t;
+  const cint *plid = (const cint *)p.point_lid;
+  const clong *prow = (const clong *)p.rowptr;
+  // part 0: class (0,0); 1: (1,0) and (1,1); 2: (0,1).  The longest part's workgroups start first.
+  const int nw = static_cast<int>(gridDim.x) / 3, part = static_cast<int>(blockIdx.x) / nw, wi = static_cast<int>(blockIdx.x) % nw;
+  const int line = wi / gp.nchunk, ck = wi % gp.nchunk;
+  const int LY = line % (p.ny + 1), LZ = line / (p.ny + 1);
+  const int x0 = ck * gp.chunk, x1 = min(x0 + gp.chunk, p.nx);
+  if (x0 >= x1) return;
+  for (int cls = part; cls < 4; cls += part == 1 ? 2 : 4) {   // bit 0: py, bit 1: pz
+    const int qy = cls & 1, qz = cls >> 1;
+    if ((qy && LY == p.ny) || (qz && LZ == p.nz)) continue;
+    const int ry = qy ? 1 : 2, rz = qz ? 1 : 2;            // reach of the nodes' neighbours
+    const int Dy = 2 * ry + 1, Dz = 2 * rz + 1, n9 = Dy * Dz * 9;
+    double *cur = mem, *mid = cur + 5 * n9, *nxt = mid + 3 * n9;
+    for (int k = lane; k < 11 * n9; k += 64) cur[k] = 0.0;
+    // cells around the line: y in [cy0, cy1], z in [cz0, cz1]
+    const int cy0 = qy ? LY : max(LY - 1, 0), cy1 = min(LY, p.ny - 1);
+    const int cz0 = qz ? LZ : max(LZ - 1, 0), cz1 = min(LZ, p.nz - 1);
+    const int my = cy1 - cy0 + 1, nc = my * (cz1 - cz0 + 1);
+    const int xs = x0 > 0 ? x0 - 1 : 0;                    // the cell before the chunk: its upper nodes
+    const int nunit = (x1 - xs) * nc;
+    // a cell's points and state are loaded while the blocks of the cell before are added to the rows, its
+    // nodes' LIDs one cell earlier
+    int32_t Ln;
+    double tn[7], un[3], mn[3], En;
+    auto cell_of = [&](int u, int &x, int &y, int &z) {
+      const int uc = min(u, nunit - 1), c = uc % nc;
+      x = xs + uc / nc;
+      y = cy0 + c % my;
+      z = cz0 + c / my;
+    };
+    auto load_lid = [&](int u) {
+      int x, y, z;
+      cell_of(u, x, y, z);
+      const int32_t *l = p.point_lid + 6 * (x + px * (y + py * z));
+      Ln = l[lo];
+    };
+    auto load_data = [&](int u) {
+      int x, y, z;
+      cell_of(u, x, y, z);
+      const int64_t c = x + static_cast<int64_t>(p.nx) * (y + static_cast<int64_t>(p.ny) * z);
+      const double *s = gp.pts + c * (27 * 16);
+#pragma unroll
+      for (int ks = 0; ks < 7; ++ks) tn[ks] = s[lane + 64 * ks];   // lane 16 g + e: entry e of point 4 ks + g (27: past the cell)
+      En = p.coef[c];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        un[j] = p.x[Ln + j];
+        mn[j] = 0.0;
+        if constexpr (TR) {
+          const double v = p.xdot[Ln + j], a = tra ? p.xddot[Ln + j] : 0.0;
+          un[j] += p.rb * v;
+          mn[j] = p.ra * v + a;
+        }
+      }
+    };
+    load_lid(0);
+    load_data(0);
+    load_lid(1);
+    double rr[3] = {0.0, 0.0, 0.0}, carry[3] = {0.0, 0.0, 0.0}, msum = 0.0;
+    int u = 0;
+    for (int x = xs; x < x1; ++x) {
+      // where the step's finished nodes go
+      const int P0 = 2 * x + px * (2 * LY + qy + py * (2 * LZ + qz));
+      const int32_t Lc = plid[3 * P0], Lm = plid[3 * P0 + 3];
+      const int64_t basec = prow[Lc], basem = prow[Lm];
+      const int lenc = static_cast<int>(prow[Lc + 1] - basec), lenm = static_cast<int>(prow[Lm + 1] - basem);
+      const uint16_t *npc = p.nperm + static_cast<int64_t>(Lc / 3) * p.nperm_w, *npm = p.nperm + static_cast<int64_t>(Lm / 3) * p.nperm_w;
+      int nc0 = npc[lane], nc1 = npc[lane + 64], nm0 = npm[lane], nm1 = npm[lane + 64];   // nperm_w = 128
+      for (int c = 0; c < nc; ++c, ++u) {
+        const int ay = qy ? 1 : 2 * (LY - cy0 - c % my), az = qz ? 1 : 2 * (LZ - cz0 - c / my);
+        if (g == 3) tn[6] = 0.0;   // 27 points: no 28th
+        if (lane < 27)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            st[lane][j] = un[j];
+            if constexpr (TR) st[lane][3 + j] = mn[j];
+          }
+        const double E = En;
+        gather_lds_sync();
+        v4d acc[2][3], accm[2];
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+          accm[cb] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+          for (int j = 0; j < 3; ++j) acc[cb][j] = v4d{0.0, 0.0, 0.0, 0.0};
+        }
+        double ml = 0.0;
+        int gq = g;
+        const double *ta = &TA[ay + 3 * az][0][0];
+#pragma unroll
+        for (int ks = 0; ks < 7; ++ks) {
+          asm volatile("" : "+v"(gq), "+v"(ml));   // a k-step's operands in registers at a time
+          const int qyz = ks < 6 ? (4 * ks + gq) * 11 >> 5 : 8;   // the point's index over y and z
+          const double yz = ta[qyz], dz_ = ta[9 + qyz], zd = ta[18 + qyz];
+          const double t = tn[ks];
+          // rows 0-2: s C dN_a; row 3: w det, 0, 0, 1 with N_a first
+          const double A = quad_entry<3>(t) * (quad_entry<0>(t) * (xd[ks % 3] * yz) + quad_entry<1>(t) * (xa[ks % 3] * dz_) +
+                                               quad_entry<2>(t) * (xa[ks % 3] * zd));
+          ml += A;
+          const double C[9] = {row_entry<0>(t), row_entry<1>(t), row_entry<2>(t), row_entry<4>(t), row_entry<5>(t),
+                               row_entry<6>(t), row_entry<8>(t), row_entry<9>(t), row_entry<10>(t)};
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) {
+            const double *d = dB[cb][ks];
+            acc[cb][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, C[0] * d[0] + C[1] * d[1] + C[2] * d[2], acc[cb][0], 0, 0, 0);
+            acc[cb][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, C[3] * d[0] + C[4] * d[1] + C[5] * d[2], acc[cb][1], 0, 0, 0);
+            acc[cb][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, C[6] * d[0] + C[7] * d[1] + C[8] * d[2], acc[cb][2], 0, 0, 0);
+            if constexpr (TR) {   // the mass columns N_b, from the 1D tables: registers hold no more
+              const int qt = ks < 6 ? 4 * ks + gq : 24 + min(gq, 2), qz_ = (qt * 57) >> 9;   // qt / 9
+              const double N = T1[3 * bo[cb][0] + qt - 3 * qyz].x * T1[3 * bo[cb][1] + qyz - 3 * qz_].x * T1[3 * bo[cb][2] + qz_].x;
+              accm[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, N, accm[cb], 0, 0, 0);
+            }
+          }
+        }
+        // the measure takes the sign of the first point's determinant (Intrepid2 computeCellMeasure)
+        const double sg = __builtin_amdgcn_readlane(__double2hiint(tn[0]), 12) < 0 ? -1.0 : 1.0;
+        load_data(u + 1);
+        load_lid(u + 2);
+        msum += sg * ml;
+        const double lam = sg * E * lamf, mu = sg * E * muf, rho = TR ? sg * p.rho : 0.0;
+        // node a = g: 0 the current node, 1 the middle one, 2 the next; slots in dx, dy, dz
+        double *dst = g == 0 ? cur + 2 * n9 : (g == 1 ? mid : nxt);
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+          const double trs = acc[cb][0][0] + acc[cb][1][1] + acc[cb][2][2];
+          const double Mab = TR ? rho * accm[cb][3] : 0.0;
+          double jv[3][3];
+          const bool in = 16 * cb + l16 < 27;
+          const int bn = min(16 * cb + l16, 26);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            double r = 0.0;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              const double Kv = lam * acc[cb][j][i] + mu * acc[cb][i][j] + (i == j ? mu * trs : 0.0);
+              r += Kv * st[bn][j];
+              jv[i][j] = cK * Kv;
+              if (TR && i == j) {
+                jv[i][j] += cM * Mab;
+                r += Mab * st[bn][TR ? 3 + j : 0];
+              }
+            }
+            rr[i] += in ? r : 0.0;
+          }
+          if (in && g < 3) {
+            double *o = dst + bo[cb][0] * n9 + ((bo[cb][1] - ay + ry) * Dz + bo[cb][2] - az + rz) * 9;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+              for (int j = 0; j < 3; ++j) atomicAdd(&o[3 * i + j], jv[i][j]);
+          }
+        }
+      }
+      // residuals: over the row of 16 lanes, less the source load (its sums are in lanes 12 + a, + 16 ...)
+      double ms4 = msum;
+      ms4 += __shfl_xor(ms4, 16);
+      ms4 += __shfl_xor(ms4, 32);
+      const double ma = __shfl(ms4, 12 + min(g, 2));
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        double r = rr[i];
+        r += dpp_f64<0xB1, 0xf>(r);
+        r += dpp_f64<0x4E, 0xf>(r);
+        r += dpp_f64<0x141, 0xf>(r);
+        r += dpp_f64<0x140, 0xf>(r);
+        r = (carry[i] + r) - p.src[i] * ma;
+        rr[i] = r;
+        carry[i] = __shfl(r, (lane & 15) + 32);   // the next node's, for lanes of row 0
+        if (g != 0) carry[i] = 0.0;
+      }
+      msum = 0.0;
+      // everything loaded is here before the stores go out: one counter tracks loads and stores
+#pragma unroll
+      for (int ks = 0; ks < 7; ++ks) asm volatile("" : "+v"(tn[ks]));
+#pragma unroll
+      for (int j = 0; j < 3; ++j) asm volatile("" : "+v"(un[j]), "+v"(mn[j]));
+      asm volatile("" : "+v"(Ln), "+v"(En), "+v"(nc0), "+v"(nc1), "+v"(nm0), "+v"(nm1));
+      gather_lds_sync();
+      if (x >= x0) {
+        if (p.f && l16 < 3 && g < 2) p.f[(g ? Lm : Lc) + l16] = l16 == 0 ? rr[0] : (l16 == 1 ? rr[1] : rr[2]);
+        store_node27(cur, inv, 2, ry, rz, nc0, nc1, p.vals, basec, lenc, lane);
+        store_node27(mid, inv, 1, ry, rz, nm0, nm1, p.vals, basem, lenm, lane);
+        gather_lds_sync();
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) rr[i] = 0.0;
+      for (int k = lane; k < 3 * n9; k += 64) {
+        cur[k] = nxt[k];
+        nxt[k] = 0.0;
+        mid[k] = 0.0;
+      }
+      for (int k = 3 * n9 + lane; k < 5 * n9; k += 64) cur[k] = 0.0;
+      gather_lds_sync();
+    }
+    if (x1 == p.nx) {   // the line's last node has no cell above
+      const int P0 = 2 * p.nx + px * (2 * LY + qy + py * (2 * LZ + qz));
+      const int32_t Lc = plid[3 * P0];
+      const int64_t basec = prow[Lc];
+      const int lenc = static_cast<int>(prow[Lc + 1] - basec);
+      const uint16_t *npc = p.nperm + static_cast<int64_t>(Lc / 3) * p.nperm_w;
+      const int n0 = npc[lane], n1 = npc[lane + 64];
+      if (p.f && l16 < 3 && g == 0) p.f[Lc + l16] = l16 == 0 ? carry[0] : (l16 == 1 ? carry[1] : carry[2]);
+      store_node27(cur, inv, 2, ry, rz, n0, n1, p.vals, basec, lenc, lane);
+      gather_lds_sync();
+    }
+  }
+}
+
 template <int NB, int NQ, int BS, int MODE>
 void launch(const ElasticParams &p, hipStream_t s) {
   int dev = 0, ncu = 0;
@@ -1826,6 +2214,11 @@ bool affine_hex8(const Mesh &m) {
 bool general_hex8(const Mesh &m, int precision) {
   if (m.topo != TXA_HEX8 || m.nfields != 3 || precision != TXA_FP64) return false;
   return m.structured ? !m.affine : m.uocc.p != nullptr;   // three int32 LIDs per point: under 2^31 points
+}
+
+// hex27 bricks in FP64 take the line kernel where the matrix is wanted
+bool line_hex27(const Mesh &m, int precision, bool want_vals) {
+  return m.topo == TXA_HEX27 && m.structured && m.nfields == 3 && precision == TXA_FP64 && want_vals;
 }
 
 // Streams and events of the element / gather slab pipeline, one set per host thread and device
@@ -1871,6 +2264,7 @@ bool elastic_supported(const Mesh &m, const txa_assembly_args &a) {
 size_t elastic_workspace_bytes(const Mesh &m, int precision, bool want_f, bool want_vals, bool footprint) {
   size_t r = 0, j = 0;
   if (affine_hex8(m) || (!footprint && general_hex8(m, precision))) return 0;
+  if (!footprint && line_hex27(m, precision, want_vals)) return ws_round(static_cast<size_t>(m.nelem) * 27 * 16 * sizeof(double) + 16 * sizeof(double));
   ws_parts(m, precision, want_f, want_vals, &r, &j);
   return r + j;
 }
@@ -2013,6 +2407,34 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
       hipLaunchKernelGGL(k_elastic8_upload<true>, dim3(resident_grid(k_elastic8_upload<true>, pairs, 64)), dim3(64), 0, s, q);
     else
       hipLaunchKernelGGL(k_elastic8_upload<false>, dim3(resident_grid(k_elastic8_upload<false>, pairs, 64)), dim3(64), 0, s, q);
+    TXA_HIP(hipGetLastError());
+    return;
+  }
+  if (line_hex27(m, a.precision, a.vals != nullptr)) {
+    TXA_REQUIRE(ws != nullptr, TXA_ERR_LOGIC, "elasticity assembly needs its workspace");
+    Node27Params q;
+    q.p = elastic8_params(m, a);
+    q.pts = static_cast<const double *>(ws);
+    const int64_t lines = static_cast<int64_t>(m.ny + 1) * (m.nz + 1);
+    const bool tr = a.transient && a.xdot;
+    // x positions per workgroup: the mean load of a wave (nine units per position and line, one more
+    // position per part of a split line) and half of the longest workgroup, which may start last
+    const double slots = tr ? resident_grid(k_elastic27_nodes<true>, INT32_MAX, 64) : resident_grid(k_elastic27_nodes<false>, INT32_MAX, 64);
+    double best = 1e300;
+    q.chunk = m.nx;
+    for (int k = 1; k <= m.nx && k <= 32; ++k) {
+      const int len = (m.nx + k - 1) / k, n = (m.nx + len - 1) / len, extra = n > 1;
+      const double t = std::max(1.0, 9.0 * lines * n / (4.0 * slots)) * 4.0 * (static_cast<double>(m.nx) / n + extra) + 2.0 * (len + extra);
+      if (t < best) { best = t; q.chunk = len; }
+    }
+    q.nchunk = (m.nx + q.chunk - 1) / q.chunk;
+    const int64_t np = m.nelem * 27;
+    hipLaunchKernelGGL(k_points27, dim3(static_cast<unsigned>((np + 255) / 256)), dim3(256), 0, s, m.nx, m.ny, m.nelem, m.xyz.p,
+                       m.xyz.p + m.nverts, m.xyz.p + 2 * m.nverts, static_cast<double *>(ws));
+    TXA_HIP(hipGetLastError());
+    const dim3 grid(static_cast<unsigned>(3 * lines * q.nchunk));
+    if (tr) hipLaunchKernelGGL(k_elastic27_nodes<true>, grid, dim3(64), 0, s, q);
+    else hipLaunchKernelGGL(k_elastic27_nodes<false>, grid, dim3(64), 0, s, q);
     TXA_HIP(hipGetLastError());
     return;
   }
