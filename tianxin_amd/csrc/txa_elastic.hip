@@ -1805,17 +1805,18 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
 //   T[(a,k),(b,l)] = sum_q s_q (C dN_a)_k (C dN_b)_l,   C the cofactors of J, s = w / det.
 // Operand row l % 16 = a + 4 k, columns b in two tiles per l: as lane l of the product holds D rows
 // l / 16 + 4 i, it ends up with all nine entries of the pair (a = l / 16, b = l % 16), so no Gram matrix
-// goes through LDS.  Row group 3 is w det N_a: with columns N_b it gives the mass matrix, and its sum over
-// the points the source load.  A lane holds one of the 16 values of each of its row's points (one coalesced
-// load per cell) and the operands are formed from DPP broadcasts of them and the wave's constant dN_b:
-// read from LDS instead (16 lanes the same 16 bytes), they took 61% of its cycles (1.84 ms against 1.53 at
-// 33^3).  Blocks are added in lattice order into the rows in LDS (one wave's LDS operations execute in order
+// goes through LDS.  Row group 3 is w det N_a: its sum over the points is the source load.  A lane holds one of the 16 values of each of its row's points (one coalesced
+// load per cell) and the operands are formed from DPP broadcasts of them: read from LDS instead (16 lanes
+// the same 16 bytes), they took 61% of its cycles (1.84 ms against 1.53 at 33^3).  Blocks are added in lattice order into the rows in LDS (one wave's LDS operations execute in order
 // and the lanes of one add hit distinct entries: a fixed order of sums, the same for every split of a
 // line), and rows are stored once in CRS order when their last cell is done.
 //
-// Bound by issue: of 2.6 M cycles per SIMD at 33^3 the products take 0.9 M (46% of their rows and columns
-// are used) and 218 k VALU instructions 0.87 M, at seven waves per CU (22.8 KB of LDS, 256 VGPRs).  Steady
-// FP64 33^3, against the element kernel with its 55 KB of blocks per element and the gather: 1.79 -> 1.17 ms.
+// Bound by issue: an FP64 product takes its SIMD's 64 cycles whole (a wave's VALU work, and the other
+// waves', wait for it: measured), 0.9 M of 2.6 M cycles per SIMD at 33^3 (46% of its rows and columns are
+// used), and 218 k VALU instructions 0.87 M more, at seven waves per CU (23 KB of LDS each).  FP64 33^3,
+// against the element kernel with its 55 KB of blocks per element and the gather: steady 1.79 -> 1.17 ms,
+// transient 2.16 -> 1.72 ms (with the mass matrix on the products too, 2.29 ms: it spilled); 12^3 steady
+// 225 -> 125 us, transient 263 -> 150 us, 4^3 steady 124 -> 48 us.
 // The FP32 and split-BF16 forms keep those: their results are rounded there.
 struct Node27Params {
   Elastic8Params p;
@@ -1915,8 +1916,10 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
   __shared__ double mem[kRows27];
   __shared__ double2 T1[9];          // 1D basis: value and derivative of node d at Gauss point q, [3 d + q]
   __shared__ double TA[9][3][9];     // [node y + 3 z][N N', N' N, N N of y, z][point y + 3 z]: of the row operand
-  __shared__ uint16_t inv[128];
+  __shared__ double PP[3][3][3];     // N_a N_b of two 1D nodes at the points
+  __shared__ double wdl[TR ? 28 : 1];   // the cell's w det
   __shared__ double st[27][TR ? 6 : 3];   // the cell's nodes: u + b_R v, a_R v + a
+  uint16_t *inv = reinterpret_cast<uint16_t *>(&st[0][0]);   // of store_node27, between two cells
   const int lane = threadIdx.x;
   if (threadIdx.x < 9) {
     const int d = threadIdx.x / 3;
@@ -1925,6 +1928,7 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
                              : (d == 1 ? make_double2(1.0 - xi * xi, -2.0 * xi) : make_double2(0.5 * xi * (xi + 1.0), xi + 0.5));
   }
   __syncthreads();
+  if (TR && lane < 27) PP[lane / 9][lane / 3 % 3][lane % 3] = T1[3 * (lane / 9) + lane % 3].x * T1[3 * (lane / 3 % 3) + lane % 3].x;
   for (int i = lane; i < 81; i += 64) {
     const int n = i / 9, q = i % 9;
     const double2 y = T1[3 * (n % 3) + q % 3], z = T1[3 * (n / 3) + q / 3];
@@ -1936,30 +1940,28 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
   const int px = 2 * p.nx + 1, py = 2 * p.ny + 1;
   const int l16 = lane & 15, g = lane >> 4;
   const int ka = l16 >> 2, ax = min(l16 & 3, 2);   // operand row: node ax, component ka (3: the mass row)
-  // nodes of this lane's columns, their lattice offsets and constant gradients at the points 4 ks + g
+  // nodes of this lane's columns: lattice offsets, and x basis and derivative at point 4 ks + g, of index
+  // (ks + g) % 3 along x: entry ks % 3 (the y and z factors come from TA)
   int bo[2][3];
-  double dB[2][7][3];
+  double xb[2][3], xbd[2][3];
 #pragma unroll
   for (int cb = 0; cb < 2; ++cb) {
-    const int b = min(16 * cb + l16, 26);   // any order of the 27 nodes: x fastest
+    const int b = min(16 * cb + l16, 26);   // x fastest
     bo[cb][0] = b % 3;
     bo[cb][1] = b / 3 % 3;
     bo[cb][2] = b / 9;
 #pragma unroll
-    for (int ks = 0; ks < 7; ++ks) {
-      const int q = min(4 * ks + g, 26);
-      const double2 x = T1[3 * bo[cb][0] + q % 3], y = T1[3 * bo[cb][1] + q / 3 % 3], z = T1[3 * bo[cb][2] + q / 9];
-      dB[cb][ks][0] = x.y * y.x * z.x;
-      dB[cb][ks][1] = x.x * y.y * z.x;
-      dB[cb][ks][2] = x.x * y.x * z.y;
-#pragma unroll
-      for (int m = 0; m < 3; ++m) asm volatile("" : "+v"(dB[cb][ks][m]));
+    for (int r = 0; r < 3; ++r) {
+      const double2 x = T1[3 * bo[cb][0] + (r + g) % 3];
+      xb[cb][r] = x.x;
+      xbd[cb][r] = x.y;
+      asm volatile("" : "+v"(xb[cb][r]), "+v"(xbd[cb][r]));
     }
   }
   // node min(lane, 26)'s LID entry from the cell's first
   const int bl = min(lane, 26);
   const unsigned lo = 3 * (bl % 3 + px * (bl / 3 % 3 + py * (bl / 9)));
-  // the row node's x basis at point 4 ks + g, of index (ks + g) % 3 along x: entry ks % 3
+  // the row node's
   double xa[3], xd[3];
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
@@ -1996,10 +1998,10 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
     const int my = cy1 - cy0 + 1, nc = my * (cz1 - cz0 + 1);
     const int xs = x0 > 0 ? x0 - 1 : 0;                    // the cell before the chunk: its upper nodes
     const int nunit = (x1 - xs) * nc;
-    // a cell's points and state are loaded while the blocks of the cell before are added to the rows, its
-    // nodes' LIDs one cell earlier
+    // a cell's points and state are loaded while the cell before is computed, its nodes' LIDs one cell
+    // earlier; a point's register takes the next cell's once its operands are formed
     int32_t Ln;
-    double tn[7], un[3], mn[3], En;
+    double tn[7], un[3], vn[3], an[3], En;
     auto cell_of = [&](int u, int &x, int &y, int &z) {
       const int uc = min(u, nunit - 1), c = uc % nc;
       x = xs + uc / nc;
@@ -2012,27 +2014,27 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
       const int32_t *l = p.point_lid + 6 * (x + px * (y + py * z));
       Ln = l[lo];
     };
-    auto load_data = [&](int u) {
+    auto points_of = [&](int u) {
       int x, y, z;
       cell_of(u, x, y, z);
-      const int64_t c = x + static_cast<int64_t>(p.nx) * (y + static_cast<int64_t>(p.ny) * z);
-      const double *s = gp.pts + c * (27 * 16);
-#pragma unroll
-      for (int ks = 0; ks < 7; ++ks) tn[ks] = s[lane + 64 * ks];   // lane 16 g + e: entry e of point 4 ks + g (27: past the cell)
-      En = p.coef[c];
+      return gp.pts + (x + static_cast<int64_t>(p.nx) * (y + static_cast<int64_t>(p.ny) * z)) * (27 * 16);
+    };
+    auto load_state = [&](int u) {
+      int x, y, z;
+      cell_of(u, x, y, z);
+      En = p.coef[x + static_cast<int64_t>(p.nx) * (y + static_cast<int64_t>(p.ny) * z)];
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         un[j] = p.x[Ln + j];
-        mn[j] = 0.0;
-        if constexpr (TR) {
-          const double v = p.xdot[Ln + j], a = tra ? p.xddot[Ln + j] : 0.0;
-          un[j] += p.rb * v;
-          mn[j] = p.ra * v + a;
-        }
+        vn[j] = TR ? p.xdot[Ln + j] : 0.0;
+        an[j] = tra ? p.xddot[Ln + j] : 0.0;
       }
     };
+    const double *pn = points_of(0);
+#pragma unroll
+    for (int ks = 0; ks < 7; ++ks) tn[ks] = pn[lane + 64 * ks];   // lane 16 g + e: entry e of point 4 ks + g (27: past the cell)
     load_lid(0);
-    load_data(0);
+    load_state(0);
     load_lid(1);
     double rr[3] = {0.0, 0.0, 0.0}, carry[3] = {0.0, 0.0, 0.0}, msum = 0.0;
     int u = 0;
@@ -2050,15 +2052,37 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
         if (lane < 27)
 #pragma unroll
           for (int j = 0; j < 3; ++j) {
-            st[lane][j] = un[j];
-            if constexpr (TR) st[lane][3 + j] = mn[j];
+            st[lane][j] = TR ? un[j] + p.rb * vn[j] : un[j];
+            if constexpr (TR) st[lane][3 + j] = p.ra * vn[j] + an[j];
           }
+        if (TR && l16 == 12)
+#pragma unroll
+          for (int ks = 0; ks < 7; ++ks) wdl[4 * ks + g] = tn[ks];
         const double E = En;
         gather_lds_sync();
-        v4d acc[2][3], accm[2];
+        load_state(u + 1);
+        load_lid(u + 2);
+        pn = points_of(u + 1);
+        // the measure takes the sign of the first point's determinant (Intrepid2 computeCellMeasure)
+        const double sg = __builtin_amdgcn_readlane(__double2hiint(tn[0]), 12) < 0 ? -1.0 : 1.0;
+        double Mb[2] = {0.0, 0.0};
+        if constexpr (TR) {   // sum_q w det N_a N_b, an axis at a time
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) {
+            const double *x = PP[min(g, 2)][bo[cb][0]], *y = PP[ay][bo[cb][1]], *z = PP[az][bo[cb][2]];
+            const double x0 = x[0], x1 = x[1], x2 = x[2], y0 = y[0], y1 = y[1], y2 = y[2];
+#pragma unroll
+            for (int qz = 0; qz < 3; ++qz) {
+              asm volatile("" : "+v"(Mb[cb]) : : "memory");   // nine weights in registers at a time
+              const double *w = wdl + 9 * qz;
+              Mb[cb] += z[qz] * (y0 * (x0 * w[0] + x1 * w[1] + x2 * w[2]) + y1 * (x0 * w[3] + x1 * w[4] + x2 * w[5]) +
+                                 y2 * (x0 * w[6] + x1 * w[7] + x2 * w[8]));
+            }
+          }
+        }
+        v4d acc[2][3];
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
-          accm[cb] = v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
           for (int j = 0; j < 3; ++j) acc[cb][j] = v4d{0.0, 0.0, 0.0, 0.0};
         }
@@ -2071,6 +2095,7 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
           const int qyz = ks < 6 ? (4 * ks + gq) * 11 >> 5 : 8;   // the point's index over y and z
           const double yz = ta[qyz], dz_ = ta[9 + qyz], zd = ta[18 + qyz];
           const double t = tn[ks];
+          tn[ks] = pn[lane + 64 * ks];
           // rows 0-2: s C dN_a; row 3: w det, 0, 0, 1 with N_a first
           const double A = quad_entry<3>(t) * (quad_entry<0>(t) * (xd[ks % 3] * yz) + quad_entry<1>(t) * (xa[ks % 3] * dz_) +
                                                quad_entry<2>(t) * (xa[ks % 3] * zd));
@@ -2079,21 +2104,13 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
                                row_entry<6>(t), row_entry<8>(t), row_entry<9>(t), row_entry<10>(t)};
 #pragma unroll
           for (int cb = 0; cb < 2; ++cb) {
-            const double *d = dB[cb][ks];
+            const double *tb = &TA[bo[cb][1] + 3 * bo[cb][2]][0][0];
+            const double d[3] = {xbd[cb][ks % 3] * tb[qyz], xb[cb][ks % 3] * tb[9 + qyz], xb[cb][ks % 3] * tb[18 + qyz]};
             acc[cb][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, C[0] * d[0] + C[1] * d[1] + C[2] * d[2], acc[cb][0], 0, 0, 0);
             acc[cb][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, C[3] * d[0] + C[4] * d[1] + C[5] * d[2], acc[cb][1], 0, 0, 0);
             acc[cb][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, C[6] * d[0] + C[7] * d[1] + C[8] * d[2], acc[cb][2], 0, 0, 0);
-            if constexpr (TR) {   // the mass columns N_b, from the 1D tables: registers hold no more
-              const int qt = ks < 6 ? 4 * ks + gq : 24 + min(gq, 2), qz_ = (qt * 57) >> 9;   // qt / 9
-              const double N = T1[3 * bo[cb][0] + qt - 3 * qyz].x * T1[3 * bo[cb][1] + qyz - 3 * qz_].x * T1[3 * bo[cb][2] + qz_].x;
-              accm[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, N, accm[cb], 0, 0, 0);
-            }
           }
         }
-        // the measure takes the sign of the first point's determinant (Intrepid2 computeCellMeasure)
-        const double sg = __builtin_amdgcn_readlane(__double2hiint(tn[0]), 12) < 0 ? -1.0 : 1.0;
-        load_data(u + 1);
-        load_lid(u + 2);
         msum += sg * ml;
         const double lam = sg * E * lamf, mu = sg * E * muf, rho = TR ? sg * p.rho : 0.0;
         // node a = g: 0 the current node, 1 the middle one, 2 the next; slots in dx, dy, dz
@@ -2101,7 +2118,7 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
           const double trs = acc[cb][0][0] + acc[cb][1][1] + acc[cb][2][2];
-          const double Mab = TR ? rho * accm[cb][3] : 0.0;
+          const double Mab = TR ? rho * Mb[cb] : 0.0;
           double jv[3][3];
           const bool in = 16 * cb + l16 < 27;
           const int bn = min(16 * cb + l16, 26);
@@ -2151,7 +2168,7 @@ __global__ __launch_bounds__(64, 2) void k_elastic27_nodes(Node27Params gp) {
 #pragma unroll
       for (int ks = 0; ks < 7; ++ks) asm volatile("" : "+v"(tn[ks]));
 #pragma unroll
-      for (int j = 0; j < 3; ++j) asm volatile("" : "+v"(un[j]), "+v"(mn[j]));
+      for (int j = 0; j < 3; ++j) asm volatile("" : "+v"(un[j]), "+v"(vn[j]), "+v"(an[j]));
       asm volatile("" : "+v"(Ln), "+v"(En), "+v"(nc0), "+v"(nc1), "+v"(nm0), "+v"(nm1));
       gather_lds_sync();
       if (x >= x0) {
