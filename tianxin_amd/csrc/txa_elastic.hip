@@ -84,17 +84,17 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-// bf16 with round-to-nearest-even (finite inputs), returned as its bit pattern and its value
+// bf16 with round-to-nearest-even, returned as its bit pattern and its value
 __device__ __forceinline__ short bf16_rne(float x, float &v) {
-  uint32_t u = __float_as_uint(x);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  const uint32_t h = u & 0xffff0000u;
-  v = __uint_as_float(h);
-  return static_cast<short>(h >> 16);
+  const __bf16 h = static_cast<__bf16>(x);   // v_cvt_pk_bf16_f32
+  const short s = __builtin_bit_cast(short, h);
+  v = __uint_as_float(static_cast<uint32_t>(static_cast<uint16_t>(s)) << 16);
+  return s;
 }
 
 // x = x0 + x1 + x2 with bf16 parts (exact up to ~2^-24 |x|)
 __device__ __forceinline__ void split3(float x, short &s0, short &s1, short &s2) {
+  asm("" : "+v"(x));   // rounded to FP32 first: converted straight from FP64, x0 differs now and then
   float v0, v1, v2;
   s0 = bf16_rne(x, v0);
   const float r1 = x - v0;
@@ -163,6 +163,7 @@ struct Smem {
   double sw[NQ];             // sqrt(w |det J|)
   double u[D::ND], v[D::ND], a[D::ND], r[D::ND];
   TReal M[NB][NB];
+  double fa[3][NB];          // integral of each basis function, by plane of points
   // VALU modes: gradients G and the Gram matrix T.  MFMA mode: the bf16 operand
   // parts, then T over the same bytes once the products are in registers.  The
   // operand rows are read as 8-byte vectors: the union is 16-byte aligned whatever
@@ -187,11 +188,13 @@ struct Smem {
   } w;
 };
 
-// The MFMA form is held to four waves per SIMD (at most 128 registers, AGPRs included),
-// which its LDS also allows: four workgroups per CU (Q2 64^3 split form 9.21 -> 8.81 ms
-// against three, at the cost of a 20-byte spill).
+// Bound by VALU issue and, beside the gather, by the block stores.  The FP32 and split hex27 forms are held
+// to three waves per SIMD (162 VGPRs; at four, 128 and 29 spilled, the split form takes 7.93 ms).  64^3
+// with the gather, against blocks staged in LDS and copied out after the pair phase, five-step sums of
+// every residual value, the source load per DOF by one thread and the bf16 parts by integer rounding:
+// split 7.86 -> 7.18 ms, FP32 8.34 -> 7.66 ms (its own stores cached: 8.33 ms).
 template <int NB, int NQ, int BS, int MODE>
-__global__ __launch_bounds__(BS, MODE == MODE_SPLIT ? 4 : 1) void k_elastic(ElasticParams p) {
+__global__ __launch_bounds__(BS, MODE == MODE_F64 || NB == 8 ? 1 : 3) void k_elastic(ElasticParams p) {
   using D = Dims<NB>;
   using TReal = typename Smem<NB, NQ, MODE>::TReal;
   constexpr int ND = D::ND;
@@ -241,9 +244,9 @@ __global__ __launch_bounds__(BS, MODE == MODE_SPLIT ? 4 : 1) void k_elastic(Elas
 
   // Gather data of the element after this one, fetched while this one is computed: the
   // coordinates, state and coefficient (thread t < 24: one vertex coordinate; t < ND:
-  // one DOF) once the Gram matrix is done, from the connectivity and LIDs fetched one
-  // element earlier; they are put in LDS after the pair phase, before the block store.
-  // No global load is then pending when the block store goes out, so the next element
+  // one DOF) beside the Gram matrix, from the connectivity and LIDs fetched one element
+  // earlier; they are waited for before the pair phase and put in LDS after it.
+  // No global load is then pending when the block stores go out, so the next element
   // starts without waiting for those stores (one counter tracks both).  The loads have
   // no branch (indices clamped to a valid element and lane; the extra values are not
   // used): a conditional load would be copied, and so waited for, where the branch joins.
@@ -335,6 +338,20 @@ __global__ __launch_bounds__(BS, MODE == MODE_SPLIT ? 4 : 1) void k_elastic(Elas
     // measure w |det J| with the sign of the first point (Intrepid2 computeCellMeasure)
     const double sg = sm.det[0] < 0.0 ? -1.0 : 1.0;
     if (t < NQ) sm.sw[t] = sqrt(sg * sm.wm[t]);
+    if (has_src)
+      for (int i = t; i < Q1 * NB; i += BS) {
+        const int a = i % NB, qz = i / NB;
+        const double *bx = sm.bL[sm.off[a][0]], *by = sm.bL[sm.off[a][1]];
+        double F = 0.0;
+#pragma unroll
+        for (int qy = 0; qy < Q1; ++qy) {
+          double l = 0.0;
+#pragma unroll
+          for (int qx = 0; qx < Q1; ++qx) l += sm.wm[(qz * Q1 + qy) * Q1 + qx] * bx[qx];
+          F += l * by[qy];
+        }
+        sm.fa[qz][a] = F * sm.bL[sm.off[a][2]][qz];
+      }
     // mass matrix (inertia and Rayleigh terms only)
     if (tr)
       for (int i = t; i < NB * NB; i += BS) {
@@ -420,6 +437,8 @@ __global__ __launch_bounds__(BS, MODE == MODE_SPLIT ? 4 : 1) void k_elastic(Elas
       }
     }
     __syncthreads();
+    fetch_data(e + gridDim.x);
+    fetch_index(e + 2 * static_cast<int64_t>(gridDim.x));
     // ---- gradient Gram matrix T
     if constexpr (MODE == MODE_SPLIT) {
       constexpr int NT = D::MP / 16;                 // 16x16 tiles per side
@@ -558,14 +577,17 @@ __global__ __launch_bounds__(BS, MODE == MODE_SPLIT ? 4 : 1) void k_elastic(Elas
       }
     }
     __syncthreads();
-    fetch_data(e + gridDim.x);
-    fetch_index(e + 2 * static_cast<int64_t>(gridDim.x));
-    // ---- 3x3 blocks of node pairs: residual rows, Jacobian values written over the
-    // pair's own T entries (the block of (a, b) depends only on those nine values)
+    // ---- 3x3 blocks of node pairs: residual rows, Jacobian values to the workspace, node-major (node
+    // a: rows i NB + a, i = 0..2, of the Gram layout; the padding is not written): the lanes of a node
+    // on consecutive entries
     //   K_ij = lambda T[(i,a),(j,b)] + mu T[(j,a),(i,b)] + delta_ij mu sum_k T[(k,a),(k,b)]
     const double lam = E * p.nu / ((1.0 + p.nu) * (1.0 - 2.0 * p.nu));
     const double mu = E / (2.0 * (1.0 + p.nu));
-    auto Tref = [&](int r, int c) -> TReal & {
+    // the next element's data is here before the block stores go out (one counter tracks both)
+    asm volatile("" : "+v"(gX), "+v"(gu), "+v"(gv), "+v"(gac), "+v"(gE), "+v"(gn), "+v"(gL));
+    constexpr int NP = block_stride(NB);
+    double rp[NPASS][3];
+    auto Tref = [&](int r, int c) -> TReal {
       if constexpr (MODE == MODE_SPLIT) return sm.w.T32[r][c];
       else return sm.w.v.T[r][c];
     };
@@ -602,43 +624,57 @@ __global__ __launch_bounds__(BS, MODE == MODE_SPLIT ? 4 : 1) void k_elastic(Elas
               jv += cM * Mab;
               rr[i] += Mab * mt[j];
             }
-            Tref(i * NB + a, j * NB + b) = static_cast<TReal>(jv);
+            if (p.jbuf) {
+              TReal *o = &static_cast<TReal *>(p.jbuf)[(e * NB + a) * NP + i * ND + j * NB + b];
+              // hex27 blocks stream past the caches (measured faster); hex8 blocks as plain stores
+              if (NB == 27) __builtin_nontemporal_store(static_cast<TReal>(jv), o);
+              else *o = static_cast<TReal>(jv);
+            }
           }
       }
-      // row residuals: fixed-order reduction over the group's b (lanes b >= NB add 0)
-      static_assert(GW == 8 || GW == 32, "group width");
 #pragma unroll
-      for (int i = 0; i < 3; ++i) rr[i] = group_sum<GW>(rr[i]);
-      if (a < NB && b == (GW == 32 ? 16 : 0))
+      for (int i = 0; i < 3; ++i) rp[k][i] = rr[i];
+    }
+    // row residuals: fixed-order reduction over each group's b (lanes b >= NB add 0)
+    static_assert(GW == 8 || GW == 32, "group width");
+    if constexpr (GW == 32) {
+      // the lanes' twelve values (pass, i) together, halved as the lanes they are summed over are: value
+      // 4 m + 2 h + r ends in the lanes of row parity r, half row h
+      static_assert(NPASS == 4, "twelve values");
+      const double *v = &rp[0][0];
+      double u6[6], u3[3];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) sm.r[3 * a + i] = rr[i];
+      for (int j = 0; j < 6; ++j) {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v[2 * j]), __double2loint(v[2 * j + 1]), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v[2 * j]), __double2hiint(v[2 * j + 1]), false, false);
+        u6[j] = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+      }
+      const bool h8 = lane & 8;
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        const double keep = h8 ? u6[2 * m + 1] : u6[2 * m], send = h8 ? u6[2 * m] : u6[2 * m + 1];
+        u3[m] = group_sum<8>(keep + dpp_f64<0x128, 0xf>(send));   // row_ror:8
+        const int val = 4 * m + 2 * (h8 ? 1 : 0) + ((lane >> 4) & 1), a = ga + val / 3 * AP;
+        if ((lane & 7) == 0 && a < NB) sm.r[3 * a + val % 3] = u3[m];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < NPASS; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const double r = group_sum<GW>(rp[k][i]);
+          if (ga + k * AP < NB && gb == 0) sm.r[3 * (ga + k * AP) + i] = r;
+        }
     }
     __syncthreads();
     put_data();   // the next element's vertices and state (LDS X, u, v, a are free now)
-    // ---- element block to the workspace, node-major (node a: rows i NB + a, i = 0..2, of
-    // the Gram layout, then padding): consecutive lanes on consecutive entries
-    if (p.jbuf) {
-      constexpr int NP = block_stride(NB);
-      for (int idx = t; idx < NB * NP; idx += BS) {
-        const int a = idx / NP, q = idx % NP;
-        const TReal v = q < 3 * ND ? TReal(Tref((q / ND) * NB + a, q % ND)) : TReal(0);
-        TReal *dst = &static_cast<TReal *>(p.jbuf)[e * (NB * NP) + idx];
-        // hex27 blocks stream past the caches (measured faster); hex8 blocks as plain stores
-        if (NB == 27) __builtin_nontemporal_store(v, dst);
-        else *dst = v;
-      }
-    }
-    __syncthreads();
     if (p.rbuf)
       for (int i = t; i < ND; i += BS) {
         double F = 0.0;
         if (has_src) {
           const int a = i / 3;
-          const int ax = sm.off[a][0], ay = sm.off[a][1], az = sm.off[a][2];
-          for (int q = 0; q < NQ; ++q) {
-            const int qx = q % Q1, qy = (q / Q1) % Q1, qz = q / (Q1 * Q1);
-            F += sm.wm[q] * sm.bL[ax][qx] * sm.bL[ay][qy] * sm.bL[az][qz];
-          }
+#pragma unroll
+          for (int k = 0; k < Q1; ++k) F += sm.fa[k][a];
           // a select, not an indexed read: src[i % 3] would be a vector load from the
           // parameters, and waiting for it would wait for the block stores
           const int c = i % 3;
@@ -1805,10 +1841,12 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
 //   T[(a,k),(b,l)] = sum_q s_q (C dN_a)_k (C dN_b)_l,   C the cofactors of J, s = w / det.
 // Operand row l % 16 = a + 4 k, columns b in two tiles per l: as lane l of the product holds D rows
 // l / 16 + 4 i, it ends up with all nine entries of the pair (a = l / 16, b = l % 16), so no Gram matrix
-// goes through LDS.  Row group 3 is w det N_a: its sum over the points is the source load.  A lane holds one of the 16 values of each of its row's points (one coalesced
-// load per cell) and the operands are formed from DPP broadcasts of them: read from LDS instead (16 lanes
-// the same 16 bytes), they took 61% of its cycles (1.84 ms against 1.53 at 33^3).  Blocks are added in lattice order into the rows in LDS (one wave's LDS operations execute in order
-// and the lanes of one add hit distinct entries: a fixed order of sums, the same for every split of a
+// goes through LDS.  Row group 3 is w det N_a: its sum over the points is the source load.  A lane
+// holds one of the 16 values of each of its row's points (one coalesced load per cell) and the operands are
+// formed from DPP broadcasts of them: read from LDS instead (16 lanes the same 16 bytes), they took 61% of
+// its cycles (1.84 ms against 1.53 at 33^3).  Blocks are added in lattice order into the rows in LDS (one
+// wave's LDS operations execute in order and the lanes of one add hit distinct entries: a fixed order of
+// sums, the same for every split of a
 // line), and rows are stored once in CRS order when their last cell is done.
 //
 // Bound by issue: an FP64 product takes its SIMD's 64 cycles whole (a wave's VALU work, and the other
