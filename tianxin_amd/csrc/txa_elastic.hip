@@ -2579,9 +2579,12 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
   // on another once that slab (and the one below) is done, so the element kernel (bound by
   // its per-element latency and VALU) of slab k+1 runs beside the gather (bound by HBM) of
   // slab k.  Node plane st*z1 at a slab's top needs the next slab: the next gather takes it.
-  // A stream under graph capture (or a brick one slab high) takes the two kernels in order
+  // A stream under graph capture (or a brick of one slab) takes the two kernels in order
   // on that stream: no streams or events are created inside a capture.
-  const int nslab = std::min(kSlabs, m.nz);
+  // A slab below some 24,000 elements costs more in launches, events and emptied CUs than the overlap
+  // gives (hex27 split, one slab against eight: 8^3 48 and 174 us, 20^3 273 and 366, 36^3 1374 and 1459;
+  // four against one and eight: 46^3 2801, 2848 and 2865 us; eight against four: 64^3 7.40 and 7.48 ms).
+  const int nslab = std::min({kSlabs, m.nz, static_cast<int>(std::min<int64_t>(m.nelem / 24000, kSlabs))});
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   TXA_HIP(hipStreamIsCapturing(s, &cs));
   if (cs != hipStreamCaptureStatusNone || nslab < 2) {
