@@ -1426,14 +1426,21 @@ __device__ __forceinline__ void row_blocks(const double *tab, int bb, int fa, do
 #pragma unroll
     for (int i = 0; i < 3; ++i) v[i] = C[i][0] * dx + C[i][1] * dy + C[i][2] * dz;
     m0 += mu;
+    // the gradients of two vertices along x differ in the sign of P and the weight of Q
+    double P[NX][3], Q[NX][3];
+#pragma unroll
+    for (int y = 0; y < NX; ++y)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        P[y][j] = C[j][0] * (gL(qy ^ y) * gL(qz));
+        Q[y][j] = __builtin_fma(C[j][2], gL(qy ^ y) * gS(qz), (y ? -1.0 : 1.0) * (C[j][1] * (gS(qy) * gL(qz))));
+      }
 #pragma unroll
     for (int k = 0; k < NBL; ++k) {
       const int rx = qx ^ (k & 1), ry = NX > 1 ? qy ^ ((k >> 1) & 1) : qy, rz = qz;
       double g[3];
 #pragma unroll
-      for (int j = 0; j < 3; ++j)
-        g[j] = C[j][0] * (gS(rx) * gL(ry) * gL(rz)) + C[j][1] * (gL(rx) * gS(ry) * gL(rz)) +
-               C[j][2] * (gL(rx) * gL(ry) * gS(rz));
+      for (int j = 0; j < 3; ++j) g[j] = __builtin_fma(Q[k >> 1][j], gL(rx), gS(rx) * P[k >> 1][j]);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -1647,7 +1654,7 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
 // 3 n + 2), 32 lanes per node: lane (element instance c of eight at a time, corner y and z) forms the
 // blocks of the two vertices along x.  Bound by latency at two waves per SIMD (245 VGPRs, 16 KB of LDS
 // per wave) and VALU issue (about 800 instructions per node: no two nodes share a point table).
-// Transient FP64, shuffled 64x61x67: 1.19 -> 0.64 ms (element kernel and gather before).  Instances come from the node's list (ascending), the row
+// Transient FP64, shuffled 64x61x67: 1.19 -> 0.63 ms (element kernel and gather before).  Instances come from the node's list (ascending), the row
 // positions from their slot maps; the blocks are added into the node's rows in LDS instance by
 // instance, so the sums have a fixed order, and the rows are stored once.
 struct Elastic8UParams {
