@@ -172,6 +172,28 @@ def _dptr(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
+def _addr(t):
+    """_dptr as an integer, for fields of the argument structures (an object less per field)."""
+    if t is None:
+        return None
+    if not t.is_cuda:
+        raise ValueError("expected a device tensor")
+    if not t.is_contiguous():
+        raise ValueError("expected a contiguous tensor")
+    return t.data_ptr()
+
+
+_DTYPES = {}   # "float64" -> torch.float64, filled on first use: the package imports without torch
+
+
+def _dtype(name):
+    d = _DTYPES.get(name)
+    if d is None:
+        import torch
+        d = _DTYPES[name] = getattr(torch, name)
+    return d
+
+
 def check_tensors(specs, device=None):
     """Raises ValueError unless every (name, tensor, dtype, n, required) of specs has the dtype
     ("float64" / "int32") and n entries (n None: any), then that every one lives on CUDA device
@@ -183,7 +205,7 @@ def check_tensors(specs, device=None):
             if required:
                 raise ValueError(f"{name} is required")
             continue
-        if str(t.dtype) != "torch." + dtype:
+        if t.dtype != _dtype(dtype):
             raise ValueError(f"{name} must be {dtype}, got {t.dtype}")
         if n is not None and t.numel() != n:
             raise ValueError(f"{name} must have {n} entries, got {t.numel()}")
@@ -192,7 +214,7 @@ def check_tensors(specs, device=None):
             continue
         if not t.is_cuda:
             raise ValueError(f"{name} must be a device tensor")
-        if device is not None and t.device.index != device:
+        if device is not None and t.get_device() != device:
             raise ValueError(f"{name} is on cuda:{t.device.index}, the engine on cuda:{device}")
 
 
@@ -211,7 +233,8 @@ def check_assembly_tensors(mesh, device, *, coef, x, f=None, vals=None, xdot=Non
 def _stream(stream):
     if stream is None:
         import torch
-        stream = torch.cuda.current_stream().cuda_stream
+        # the current stream's handle without a Stream object around it
+        stream = torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return ctypes.c_void_p(stream)
 
 
@@ -222,16 +245,15 @@ def make_args(*, physics, coef, x, f=None, vals=None, precision=FP64, xdot=None,
     with sides SIDE_BOTTOM .. SIDE_FRONT."""
     a = AssemblyArgs()
     a.physics, a.precision = physics, precision
-    a.coef = _dptr(coef)
+    a.coef = _addr(coef)
     a.nu, a.rho = nu, rho
-    s = list(src) + [0.0] * 3
-    a.src = (ctypes.c_double * 3)(*s[:3])
+    a.src[:] = (*src, 0.0, 0.0, 0.0)[:3]
     a.rayleigh_a, a.rayleigh_b = rayleigh
-    a.x, a.xdot, a.xddot = _dptr(x), _dptr(xdot), _dptr(xddot)
+    a.x, a.xdot, a.xddot = _addr(x), _addr(xdot), _addr(xddot)
     a.alpha, a.beta, a.gamma2 = alpha, beta, gamma2
     a.transient = int(transient)
-    a.f, a.vals = _dptr(f), _dptr(vals)
-    a.bc_lids, a.bc_vals = _dptr(bc_lids), _dptr(bc_vals)
+    a.f, a.vals = _addr(f), _addr(vals)
+    a.bc_lids, a.bc_vals = _addr(bc_lids), _addr(bc_vals)
     a.n_bc = 0 if bc_lids is None else int(bc_lids.numel())
     a.block, a.accumulate = int(block), int(accumulate)
     if neumann:
@@ -473,10 +495,10 @@ class Model:
                        ("x_dot_dot", x_dot_dot, "float64", m.ndofs, False), ("f", f, "float64", m.ndofs, False),
                        ("W", W, "float64", m.nnz, False)], self.eng.device)
         i = ModelIn()
-        i.x, i.x_dot, i.x_dot_dot = _dptr(x), _dptr(x_dot), _dptr(x_dot_dot)
+        i.x, i.x_dot, i.x_dot_dot = _addr(x), _addr(x_dot), _addr(x_dot_dot)
         i.alpha, i.beta, i.gamma2, i.t, i.step_size = alpha, beta, gamma2, t, step_size
         o = ModelOut()
-        o.f, o.W = _dptr(f), _dptr(W)
+        o.f, o.W = _addr(f), _addr(W)
         self.eng.check(self.eng.lib.txa_model_eval(self.eng.h, self.id, ctypes.byref(i), ctypes.byref(o),
                                                    _stream(stream)))
 
