@@ -1872,8 +1872,10 @@ struct Node27Params {
 __global__ __launch_bounds__(256) void k_points27(int nx, int ny, int64_t ncell, const double *__restrict__ X,
                                                   const double *__restrict__ Y, const double *__restrict__ Z,
                                                   double *__restrict__ pts) {
-  const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (id >= ncell * 27) return;
+  // entries staged in LDS and stored by consecutive lanes: 47 -> 27 us at 33^3 (124 MB)
+  __shared__ double out[256][17];
+  const int64_t id0 = static_cast<int64_t>(blockIdx.x) * 256, n = ncell * 27;
+  const int64_t id = min(id0 + threadIdx.x, n - 1);   // past the last point: that point again, not stored
   const int64_t c = id / 27;
   const int q = static_cast<int>(id - 27 * c), qd[3] = {q % 3, q / 3 % 3, q / 9};
   const int64_t i = c % nx, j = c / nx % ny, k = c / (static_cast<int64_t>(nx) * ny);
@@ -1911,14 +1913,21 @@ __global__ __launch_bounds__(256) void k_points27(int nx, int ny, int64_t ncell,
   C[8] = J[0][0] * J[1][1] - J[0][1] * J[1][0];
   const double det = J[0][0] * C[0] + J[0][1] * C[1] + J[0][2] * C[2];
   const double s = w / det;
-  double2 *o = reinterpret_cast<double2 *>(pts + 16 * id);
+  double *o = out[threadIdx.x];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    o[2 * k] = make_double2(C[3 * k], C[3 * k + 1]);
-    o[2 * k + 1] = make_double2(C[3 * k + 2], s);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) o[4 * k + m] = C[3 * k + m];
+    o[4 * k + 3] = s;
   }
-  o[6] = make_double2(w * det, 0.0);
-  o[7] = make_double2(0.0, 1.0);
+  o[12] = w * det;
+  o[13] = o[14] = 0.0;
+  o[15] = 1.0;
+  __syncthreads();
+  const int left = static_cast<int>(min(n - id0, int64_t(256))) * 16;
+#pragma unroll
+  for (int k = threadIdx.x; k < 4096; k += 256)
+    if (k < left) pts[16 * id0 + k] = out[k >> 4][k & 15];
 }
 
 constexpr int rows27(int n9) { return 5 * n9 + 2 * 3 * n9; }   // current, middle and next nodes of a line
