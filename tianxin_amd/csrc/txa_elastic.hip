@@ -24,8 +24,8 @@
 // each FP32 operand (x = x0 + x1 + x2, every x_s in bf16) keeping the six cross products
 // of order <= 2^-16, accumulated in FP32.
 //
-// Bricks of parallelepiped hex8 cells skip both phases: k_elastic8_affine forms each
-// node's rows directly from closed-form cell blocks (one wave per node, no workspace).
+// hex8 in FP64 (parallelepiped bricks in every precision) and hex27 bricks in FP64 with the matrix
+// skip both phases: the node and line kernels below form rows directly and need no element blocks.
 //
 // Assembly into the CRS is two-phase.  The element kernel writes each element's
 // Jacobian block (FP32, FP64 in FP64 mode) and residual (FP64) to a workspace,
@@ -2489,7 +2489,9 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
     const int64_t lines = static_cast<int64_t>(m.ny + 1) * (m.nz + 1);
     const bool tr = a.transient && a.xdot;
     // x positions per workgroup: the mean load of a wave (nine units per position and line, one more
-    // position per part of a split line) and half of the longest workgroup, which may start last
+    // position per part of a split line) and half of the longest workgroup, which may start last.
+    // Measured with 1, 2, 3, 4, 6 parts: 6^3 109, 80, 66, 66, 52 us (six chosen), 10^3 173, 115, 103, 93, 93
+    // (ten: 102), 24^3 571, 515, 508, 522, 548 (four), 33^3 1215, 1159, 1165, 1299, 1285 us (three).
     const double slots = tr ? resident_grid(k_elastic27_nodes<true>, INT32_MAX, 64) : resident_grid(k_elastic27_nodes<false>, INT32_MAX, 64);
     double best = 1e300;
     q.chunk = m.nx;
