@@ -1211,7 +1211,10 @@ __global__ __launch_bounds__(256, 3) void k_elastic8_affine(Elastic8Params p) {
     const bool cell_ok = node_ok && cx >= 0 && cx < p.nx && cy >= 0 && cy < p.ny && cz >= 0 && cz < p.nz;
     const double E = cell_ok ? En : 0.0;
     double2 G[5];
-    const double2 *gp = reinterpret_cast<const double2 *>(p.geom + 10 * static_cast<int64_t>(cell_ok ? cx + p.nx * (cy + p.ny * cz) : 0));
+    // an absent cell takes the geometry of the nearest one, which has this node and every vertex that the
+    // two share: a degenerate cell reaches the rows of its own vertices only
+    const int gx_ = min(max(cx, 0), p.nx - 1), gy_ = min(max(cy, 0), p.ny - 1), gz_ = min(max(cz, 0), p.nz - 1);
+    const double2 *gp = reinterpret_cast<const double2 *>(p.geom + 10 * static_cast<int64_t>(gx_ + p.nx * (gy_ + p.ny * gz_)));
 #pragma unroll
     for (int t = 0; t < 5; ++t) G[t] = gp[t];
     const int64_t base = p.rowptr[L0];
@@ -1291,7 +1294,7 @@ __global__ __launch_bounds__(256, 3) void k_elastic8_affine(Elastic8Params p) {
     // residual: the cell's source load enters once, then the sum over the node's 16 lanes
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      double r = rr[i] - (q.h == 0 ? p.src[i] * adet : 0.0);
+      double r = cell_ok ? rr[i] - (q.h == 0 ? p.src[i] * adet : 0.0) : 0.0;   // selected: 0 times an Inf state is NaN
       r += dpp_f64<0xB1, 0xf>(r);
       r += dpp_f64<0x4E, 0xf>(r);
       r += dpp_f64<0x141, 0xf>(r);
@@ -1605,7 +1608,7 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
     // residual: the cell's source load enters once, then the sum over the node's 16 lanes
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      double r = rr[i] - (h == 0 ? p.src[i] * m0 : 0.0);
+      double r = cell_ok ? rr[i] - (h == 0 ? p.src[i] * m0 : 0.0) : 0.0;   // selected: 0 times an Inf state is NaN
       r += dpp_f64<0xB1, 0xf>(r);
       r += dpp_f64<0x4E, 0xf>(r);
       r += dpp_f64<0x141, 0xf>(r);
