@@ -93,6 +93,8 @@ __device__ __forceinline__ void walsh8_t(double (&v)[8]) {
 
 // Trilinear interpolation to the 2x2x2 Gauss points and its transpose (the matrix
 // P(a_d, q_d) is symmetric): v[q] <- sum_a prod_d P(a_d, q_d) v[a].
+// The fused products are written out: which of the two the compiler fuses depends on the kernel
+// around it, and the residual-only kernel has to give the row-owner kernel's f bit for bit.
 __device__ __forceinline__ void interp8(double (&v)[8]) {
 #pragma unroll
   for (int b = 0; b < 3; ++b)
@@ -100,8 +102,8 @@ __device__ __forceinline__ void interp8(double (&v)[8]) {
     for (int i = 0; i < 8; ++i)
       if (!bit(i, b)) {
         const double lo = v[i], hi = v[i | (1 << b)];
-        v[i] = kP * lo + kM * hi;
-        v[i | (1 << b)] = kM * lo + kP * hi;
+        v[i] = __builtin_fma(kP, lo, kM * hi);
+        v[i | (1 << b)] = __builtin_fma(kP, hi, kM * lo);
       }
 }
 
