@@ -2290,7 +2290,10 @@ bool general_hex8(const Mesh &m, int precision) {
   return m.structured ? !m.affine : m.uocc.p != nullptr;   // three int32 LIDs per point: under 2^31 points
 }
 
-// hex27 bricks in FP64 take the line kernel where the matrix is wanted
+// hex27 bricks in FP64 take the line kernel where the matrix is wanted.  f alone keeps the element kernel
+// and gather: its workspace (648 bytes per element, against the line kernel's 3456 of points) bounds the
+// sizes that calls without allocation accept, and small calls are faster (6^3 35 us against 50, 33^3 1.20
+// ms against 1.16 of the full call).  The two sum in different orders: f agrees to rounding, not bit for bit.
 bool line_hex27(const Mesh &m, int precision, bool want_vals) {
   return m.topo == TXA_HEX27 && m.structured && m.nfields == 3 && precision == TXA_FP64 && want_vals;
 }
