@@ -77,6 +77,16 @@ __device__ __forceinline__ constexpr int tet_v(int t, int j) {
   return T[t][j];
 }
 
+// whether vertices a and b share a tet (19 of the 28 pairs)
+__device__ __forceinline__ constexpr bool tet_edge(int a, int b) {
+  for (int t = 0; t < 6; ++t) {
+    int n = 0;
+    for (int j = 0; j < 4; ++j) n += tet_v(t, j) == a || tet_v(t, j) == b;
+    if (n == 2) return true;
+  }
+  return false;
+}
+
 // a b - c d and a0 b0 + a1 b1 + a2 b2 with their fused operations written out: left to the
 // compiler, which product is fused depends on what else the kernel around it uses, and the
 // residual-only kernel has to give the row-owner kernel's f bit for bit.
@@ -85,18 +95,33 @@ __device__ __forceinline__ double dot3(double a0, double b0, double a1, double b
   return __builtin_fma(a2, b2, __builtin_fma(a1, b1, a0 * b0));
 }
 
+// x / 6, correctly rounded: the product with 1/6 and its remainder (three operations, a division eleven)
+__device__ __forceinline__ double sixth(double x) {
+  const double q = x * (1.0 / 6.0);
+  return __builtin_fma(__builtin_fma(-6.0, q, x), 1.0 / 6.0, q);
+}
+
 // The six linear tets of one cell, assembled into the cell's 8x8 matrix (pairs
 // not joined by a tet edge stay zero).  Constant gradients: grad N_j = cof[:,j]/det
 // (j = 1..3), grad N_0 = -(sum); measure w |det| with w = 1/6; the degree-2
 // rule integrates the source (|T|/4 per vertex) and mass (|T|/20 (1 + delta)) exactly.
 // k: the six tet coefficients, in element order 6*cell + t.
+// Residual: FP32 takes K u from the FP64 flux of each tet; FP64 from the cell's matrix by edges,
+// K_ab (u_b - u_a), 57 operations per cell beside the matrix where the flux takes 200; without the
+// matrix its diagonal and M are not formed (100^3 steady: full call 122 -> 112 us, f alone 51 -> 49).
 template <typename Real, bool TRANS, bool UNIT, class Mid>
 __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double (&u)[8], const double (&ud)[8],
                                           const double (&k)[6], double rhoc, double src, double alpha, double beta,
                                           Hex8Out<Real, TRANS> &o, Mid &&mid) {
+  constexpr bool kFlux = flux_residual<Real>();
   mid();
   Real K[36], M[TRANS ? 36 : 1];
-  double F[8], Rf[8];   // source load; residual K u + M udot, from the flux
+  double F[8], Rf[8];   // source load; residual K u + M udot
+  double X0[3][8];   // X, FP64 form: opaque from one tet to the next
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int v = 0; v < 8; ++v) X0[d][v] = X[d][v];
 #pragma unroll
   for (int i = 0; i < 36; ++i) { K[i] = Real(0); if (TRANS) M[i] = Real(0); }
 #pragma unroll
@@ -107,7 +132,7 @@ __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double 
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
-      for (int j = 0; j < 3; ++j) J[d][j] = X[d][tet_v(t, j + 1)] - X[d][tet_v(t, 0)];
+      for (int j = 0; j < 3; ++j) J[d][j] = X0[d][tet_v(t, j + 1)] - X0[d][tet_v(t, 0)];
     double c[3][3];
     c[0][0] = diff2(J[1][1], J[2][2], J[1][2], J[2][1]);
     c[0][1] = diff2(J[1][2], J[2][0], J[1][0], J[2][2]);
@@ -120,12 +145,11 @@ __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double 
     c[2][2] = diff2(J[0][0], J[1][1], J[0][1], J[1][0]);
     const double det = dot3(J[0][0], c[0][0], J[0][1], c[0][1], J[0][2], c[0][2]);
     const double sg = det < 0.0 ? -1.0 : 1.0;
-    const double vol = det * sg / 6.0;                 // sum of the weighted measure
-    const double cw64 = k[t] * sg * recip(det) / 6.0;
+    const double vol = sixth(det * sg);                // sum of the weighted measure
+    const double cw64 = sixth(k[t] * sg * recip(det));
     const Real cw = Real(cw64);
-    {
-      // FP64: grad u (times det) = cof (u_j - u_0), R_j = cw g_j . (cof du), R_0 = -(R_1 + R_2 + R_3);
-      // mass rho_c |T| / 20 (udot_a + sum_b udot_b)
+    if constexpr (kFlux) {
+      // FP64: grad u (times det) = cof (u_j - u_0), R_j = cw g_j . (cof du), R_0 = -(R_1 + R_2 + R_3)
       const double du0 = u[tet_v(t, 1)] - u[tet_v(t, 0)], du1 = u[tet_v(t, 2)] - u[tet_v(t, 0)],
                    du2 = u[tet_v(t, 3)] - u[tet_v(t, 0)];
       double tt[3];
@@ -139,12 +163,12 @@ __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double 
         rs += r;
       }
       Rf[tet_v(t, 0)] -= rs;
-      if constexpr (TRANS) {
-        const double sud = ud[tet_v(t, 0)] + ud[tet_v(t, 1)] + ud[tet_v(t, 2)] + ud[tet_v(t, 3)];
-        const double mw = rhoc * vol * 0.05;
+    }
+    if constexpr (TRANS) {   // mass rho_c |T| / 20 (udot_a + sum_b udot_b)
+      const double sud = ud[tet_v(t, 0)] + ud[tet_v(t, 1)] + ud[tet_v(t, 2)] + ud[tet_v(t, 3)];
+      const double mw = rhoc * vol * 0.05;
 #pragma unroll
-        for (int a = 0; a < 4; ++a) Rf[tet_v(t, a)] = __builtin_fma(mw, sud + ud[tet_v(t, a)], Rf[tet_v(t, a)]);
-      }
+      for (int a = 0; a < 4; ++a) Rf[tet_v(t, a)] = __builtin_fma(mw, sud + ud[tet_v(t, a)], Rf[tet_v(t, a)]);
     }
     Real g[4][3];
 #pragma unroll
@@ -154,17 +178,39 @@ __device__ __forceinline__ void tet6_cell(const double (&X)[3][8], const double 
     }
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
-      F[tet_v(t, a)] += src * vol * 0.25;
+      if constexpr (kFlux) F[tet_v(t, a)] += src * vol * 0.25;
+      else Rf[tet_v(t, a)] = __builtin_fma(-0.25 * src, vol, Rf[tet_v(t, a)]);
 #pragma unroll
       for (int b = a; b < 4; ++b) {
-        const Real gg = g[a][0] * g[b][0] + g[a][1] * g[b][1] + g[a][2] * g[b][2];
-        K[sym8(tet_v(t, a), tet_v(t, b))] += cw * gg;
+        Real &kab = K[sym8(tet_v(t, a), tet_v(t, b))];
+        if constexpr (kFlux) kab += cw * (g[a][0] * g[b][0] + g[a][1] * g[b][1] + g[a][2] * g[b][2]);
+        else kab = __builtin_fma(cw, dot3(g[a][0], g[b][0], g[a][1], g[b][1], g[a][2], g[b][2]), kab);
         if (TRANS) M[sym8(tet_v(t, a), tet_v(t, b))] += Real(rhoc * vol * (a == b ? 0.1 : 0.05));
       }
     }
+    // FP64: one tet's gradients in registers at a time (left to itself the compiler forms all six
+    // tets' first and spills 150 registers)
+    if constexpr (!kFlux) {
+      // (vertices 0 and 7 belong to every tet)
+      asm volatile("" : "+v"(X0[0][0]), "+v"(X0[1][0]), "+v"(X0[2][0]), "+v"(X0[0][7]), "+v"(X0[1][7]), "+v"(X0[2][7]),
+                   "+v"(K[sym8(tet_v(t, 0), tet_v(t, 1))]), "+v"(K[sym8(tet_v(t, 0), tet_v(t, 2))]),
+                   "+v"(K[sym8(tet_v(t, 0), tet_v(t, 3))]), "+v"(K[sym8(tet_v(t, 1), tet_v(t, 2))]),
+                   "+v"(K[sym8(tet_v(t, 1), tet_v(t, 3))]), "+v"(K[sym8(tet_v(t, 2), tet_v(t, 3))]));
+    }
+  }
+  if constexpr (!kFlux) {
+#pragma unroll
+    for (int a = 0; a < 8; ++a)
+#pragma unroll
+      for (int b = a + 1; b < 8; ++b)
+        if (tet_edge(a, b)) {
+          const double du = u[b] - u[a];
+          Rf[a] = __builtin_fma(K[sym8(a, b)], du, Rf[a]);
+          Rf[b] = __builtin_fma(-K[sym8(a, b)], du, Rf[b]);
+        }
   }
 #pragma unroll
-  for (int a = 0; a < 8; ++a) o.R[a] = Rf[a] - F[a];
+  for (int a = 0; a < 8; ++a) o.R[a] = kFlux ? Rf[a] - F[a] : Rf[a];
 #pragma unroll
   for (int i = 0; i < 36; ++i)
     o.K[i] = TRANS ? Real(beta) * K[i] + Real(alpha) * M[i] : (UNIT ? K[i] : Real(beta) * K[i]);
