@@ -374,7 +374,7 @@ def bench_batch(args):
                      "hbm_frac": cbytes / (t / 1e3) / HBM_PEAK,
                      "tuner_best_ms": tuned_ms,
                      "slab": info["slab"], "grid": info["grid"], "work_items": info["items"],
-                     "tile": f"{info['tile_x']}x{8 if info['tile_x'] == 32 or name.startswith('fp32') else 16}", "launches": info["launches"]}
+                     "tile": f"{info['tile_x']}x{info['tile_y']}", "launches": info["launches"]}
         log(f"{name}: {t:.3f} ms (tile {info['tile_x']}, slab {info['slab']}, grid {info['grid']})")
         b.destroy()
 

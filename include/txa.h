@@ -335,9 +335,9 @@ int txa_batch_destroy(txa_ctx ctx, int batch_id);
  * as for txa_assemble).  Host-blocking only while a previous launch of the
  * same batch still reads its argument blocks. */
 int txa_batch_assemble(txa_ctx ctx, int batch_id, const txa_assembly_args *args, int use_graph, void *stream);
-/* Autotuner: times `reps` launches for each tile shape (32 x 8 or 16 x 16, in FP32 16 x 8, vertex
+/* Autotuner: times `reps` launches for each tile shape (32 x 8, 16 x 16 and in FP32 16 x 8 vertex
  * columns per workgroup), slab height (vertex layers per work item: 8, 16, 32,
- * 64, whole column) and persistent grid (1, 2, 4 workgroups per CU), keeps the
+ * 64, whole column) and persistent grid (1, 2, 4 workgroups of 512 threads per CU), keeps the
  * fastest and reports its time per launch in
  * best_ms.  The counterpart of the workset-size sweep in
  * adapters-stk/example/MixedPoissonExample/analyze_performance.py:57-61; it
@@ -345,13 +345,15 @@ int txa_batch_assemble(txa_ctx ctx, int batch_id, const txa_assembly_args *args,
 int txa_batch_tune(txa_ctx ctx, int batch_id, const txa_assembly_args *args, int reps, void *stream,
                    double *best_ms);
 /* Sets the work shape by hand instead of txa_batch_tune: tile width (16 or 32 vertex
- * columns along x; the tile is 32 x 8, or 16 x 16, in FP32 16 x 8), slab height (vertex layers per work
- * item, 0 = whole column) and persistent workgroups.  The counterpart of the "Workset
+ * columns along x; the tile is tile_x x 256/tile_x; in FP32 also 16 | 8 << 16: 16 x 8, an FP32
+ * batch's tile until it is tuned or set), slab height (vertex layers per work
+ * item, 0 = whole column) and persistent workgroups of 512 threads (a 16 x 8 tile runs two of 256
+ * for each).  The counterpart of the "Workset
  * Size" entry of the assembly parameters
  * (adapters-stk/src/Panzer_STK_ModelEvaluatorFactory_impl.hpp:294). */
 int txa_batch_shape(txa_ctx ctx, int batch_id, int tile_x, int slab, int grid);
 /* out[0]=meshes out[1]=work items out[2]=slab height (0 = whole) out[3]=persistent workgroups
- * out[4]=tile width (vertex columns along x; see txa_batch_shape)
+ * out[4]=tile (as txa_batch_shape takes it: the width, for a 16 x 8 tile 16 | 8 << 16)
  * out[5]=kernel launches per call besides the Dirichlet pass (1: both element kinds in one) */
 int txa_batch_info(txa_ctx ctx, int batch_id, int64_t *out);
 

@@ -560,15 +560,18 @@ class Batch:
                                                    ctypes.byref(ms)))
         return ms.value
 
-    def shape(self, tile_x=32, slab=0, grid=256):
-        """Sets tile width (16 or 32), slab height (0: whole column) and persistent grid by hand."""
-        self.eng.check(self.eng.lib.txa_batch_shape(self.eng.h, self.id, int(tile_x), int(slab), int(grid)))
+    def shape(self, tile_x=32, slab=0, grid=256, tile_y=0):
+        """Sets tile width (16 or 32; tile_y 0: a height of 256 / tile_x, FP32 also 16 x 8), slab height (0: whole
+        column) and persistent grid by hand."""
+        self.eng.check(self.eng.lib.txa_batch_shape(self.eng.h, self.id, int(tile_x) | int(tile_y) << 16, int(slab),
+                                                    int(grid)))
 
     def info(self):
         out = np.zeros(6, np.int64)
         self.eng.check(self.eng.lib.txa_batch_info(self.eng.h, self.id, _np(out)))
-        return dict(meshes=int(out[0]), items=int(out[1]), slab=int(out[2]), grid=int(out[3]), tile_x=int(out[4]),
-                    launches=int(out[5]))
+        tile_x = int(out[4]) & 0xffff
+        return dict(meshes=int(out[0]), items=int(out[1]), slab=int(out[2]), grid=int(out[3]), tile_x=tile_x,
+                    launches=int(out[5]), tile_y=int(out[4]) >> 16 or 256 // tile_x)
 
     def destroy(self):
         if self.id is not None:

@@ -39,8 +39,8 @@ struct Tile {
   static constexpr int NOWN = TX * (TY - 1);   // owner lanes with rows
 };
 using Wide = Tile<32, 256>;     // one workgroup per CU (LDS)
-using Square = Tile<16, 256>;   // one workgroup per CU, FP64 batches
-using Small = Tile<16, 128>;    // two workgroups per CU
+using Square = Tile<16, 256>;   // one workgroup per CU, batches
+using Small = Tile<16, 128>;    // two workgroups per CU, single meshes and FP32 batches
 using namespace q1elem;
 // element kinds of the lattice kernels: TXA_HEX8 (general trilinear cells), TXA_TET4 (six
 // tets per cell) and hex8 cells that are all parallelepipeds (constant metric per cell)
@@ -1076,9 +1076,14 @@ struct Batch {
   int precision = TXA_FP64;
   bool transient = false;
   int slab = 0;   // vertex layers per work item (0: whole column)
-  int tx = 16;    // tile width, vertex columns along x: 32 x 8; 16 x 16 (FP64), 16 x 8 (FP32)
-  int grid = 0;   // persistent workgroups
-  int tile_y() const { return tx == 32 ? Wide::TY : precision == TXA_FP32 ? Small::TY : Square::TY; }
+  // tile: 32 x 8, 16 x 16 or (FP32) 16 x 8 vertex columns
+  int tx = 16, ty = 16;
+  // persistent workgroups of 512 threads; a 16 x 8 tile (256 threads) puts two in the place of one
+  int grid = 0;
+  bool small() const { return tx == Small::TX && ty == Small::TY; }
+  unsigned workgroups(int nitems) const {
+    return static_cast<unsigned>(std::min<int64_t>(static_cast<int64_t>(grid) * (small() ? 2 : 1), nitems));
+  }
   std::vector<int> zc;
   std::vector<int4> items_h;   // hex8 items, then tet4 items
   size_t n_hex = 0;            // items of hex8 meshes (the first n_hex of items_h)
@@ -1141,7 +1146,7 @@ void batch_build_items(Batch &b, int slab) {
     const int nch = (layers + zc - 1) / zc;
     std::vector<int4> &out = lists[m.topo == TXA_TET4 ? 1 : 0];
     for (int z = 0; z < nch; ++z)
-      for (int y = 0; y < tiles_y(m, b.tile_y()); ++y)
+      for (int y = 0; y < tiles_y(m, b.ty); ++y)
         for (int x = 0; x < tiles_x(m, b.tx); ++x) out.push_back(make_int4(static_cast<int>(i), x, y, z));
   }
   auto cost = [&](const int4 &w) {
@@ -1222,11 +1227,9 @@ void launch_batch_tx(const Batch &b, dim3 g, const int4 *items, int n, BatchQueu
       else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, double, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
     }
   }
-  if constexpr (!std::is_same<T, Square>::value) {   // Square: FP64 only
-    if (b.precision == TXA_FP32) {
-      if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
-      else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
-    }
+  if (b.precision == TXA_FP32) {
+    if (b.transient) hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, true>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
+    else hipLaunchKernelGGL((k_q1_batch_spec<T, KIND, float, false>), g, dim3(T::NT), 0, s, b.prm.p, items, n, q);
   }
   TXA_HIP(hipGetLastError());
 }
@@ -1234,7 +1237,7 @@ void launch_batch_tx(const Batch &b, dim3 g, const int4 *items, int n, BatchQueu
 template <int KIND>
 void launch_batch(const Batch &b, dim3 g, const int4 *items, int n, BatchQueue *q, hipStream_t s) {
   if (b.tx == 32) launch_batch_tx<Wide, KIND>(b, g, items, n, q, s);
-  else if (b.precision == TXA_FP32) launch_batch_tx<Small, KIND>(b, g, items, n, q, s);
+  else if (b.small()) launch_batch_tx<Small, KIND>(b, g, items, n, q, s);
   else launch_batch_tx<Square, KIND>(b, g, items, n, q, s);
 }
 
@@ -1252,16 +1255,18 @@ void batch_enqueue(Batch &b, hipStream_t s, int *err) {
   const int4 *it[2] = {b.items.p, b.items.p + b.n_hex};
   if (b.mixed) {
     const int nall = static_cast<int>(b.items_h.size());
-    const dim3 g(std::min(b.grid, nall));
-    if (b.tx == 16)
+    const dim3 g(b.workgroups(nall));
+    if (b.small())
       hipLaunchKernelGGL((k_q1_batch_mixed<Small, kHex8Affine, float, false>), g, dim3(Small::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
+    else if (b.tx == 16)
+      hipLaunchKernelGGL((k_q1_batch_mixed<Square, kHex8Affine, float, false>), g, dim3(Square::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
     else
       hipLaunchKernelGGL((k_q1_batch_mixed<Wide, kHex8Affine, float, false>), g, dim3(Wide::NT), 0, s, b.prm.p, b.items.p, nall, b.q.p);
     TXA_HIP(hipGetLastError());
   }
   for (int k = 0; k < 2 && !b.mixed; ++k) {
     if (nk[k] == 0) continue;
-    const dim3 g(std::min(b.grid, nk[k]));
+    const dim3 g(b.workgroups(nk[k]));
     BatchQueue *q = b.q.p + k;
     if (k == 0 && b.hex_affine) launch_batch<kHex8Affine>(b, g, it[k], nk[k], q, s);
     else if (k == 0) launch_batch<TXA_HEX8>(b, g, it[k], nk[k], q, s);
@@ -1322,14 +1327,15 @@ Batch *batch_create(const std::vector<Mesh *> &meshes, const std::vector<int> &i
   // one recomputed layer and the start of each item counted as two, spread over them with half a
   // slab as tail, take least (4 meshes of 16-64 cells: 148 us with slabs of 32 layers, 100 with 6).
   const int slots = precision == TXA_FP32 ? 2 * ncu : ncu;
-  b->grid = slots;
+  b->grid = ncu;
+  if (precision == TXA_FP32) b->ty = Small::TY;
   int slab = 0;
   double best = 0.0;
   for (int z : {4, 6, 8, 12, 16, 24, 32, 48, 64}) {
     double steps = 0.0, longest = 0.0;
     for (const Mesh *m : meshes) {
       const int layers = m->nz + 1, zc = std::min(z, layers), chunks = (layers + zc - 1) / zc;
-      steps += static_cast<double>(tiles_x(*m, b->tx)) * tiles_y(*m, b->tile_y()) * (layers + 2 * chunks);
+      steps += static_cast<double>(tiles_x(*m, b->tx)) * tiles_y(*m, b->ty) * (layers + 2 * chunks);
       longest = std::max(longest, zc + 2.0);
     }
     const double cost = std::max(steps / slots + 0.5 * longest, longest);
@@ -1361,9 +1367,12 @@ void batch_assemble(Batch &b, const txa_assembly_args *args, bool use_graph, hip
   b.launched = true;
 }
 
-// Autotuner: times the batch over tile widths (32, 16), slab heights (the
-// analogue of Panzer's workset size sweep) and persistent grid sizes, keeps the
-// fastest.  out: best ms.
+// Autotuner: times the batch over the tiles, slab heights (the analogue of
+// Panzer's workset size sweep) and persistent grid sizes, keeps the fastest.
+// FP32 tries 16 x 16 beside 16 x 8: it is up to 9% faster where a small batch's
+// items are general hex8 cells (48 meshes of 8-48 cells, transient: 222 us against
+// 243), 16 x 8 up to 18% where there are many (512 meshes: 1.96 ms against 2.2);
+// more 16 x 8 workgroups than the resident ones never won.  out: best ms.
 double batch_tune(Batch &b, const txa_assembly_args *args, hipStream_t s, int reps, int *err) {
   int dev = 0, ncu = 0;
   TXA_HIP(hipGetDevice(&dev));
@@ -1374,15 +1383,19 @@ double batch_tune(Batch &b, const txa_assembly_args *args, hipStream_t s, int re
   TXA_HIP(hipEventCreate(&e0));
   TXA_HIP(hipEventCreate(&e1));
   double best = 1e30;
-  int best_slab = b.slab, best_grid = b.grid, best_tx = b.tx;
+  int best_slab = b.slab, best_grid = b.grid, best_tx = b.tx, best_ty = b.ty;
   if (b.launched) TXA_HIP(hipEventSynchronize(b.done));
   batch_fill(b, args);   // the argument blocks stay as they are for every timed launch
-  for (int tx : {32, 16}) {
-    b.tx = tx;
+  const int tiles[][2] = {{Wide::TX, Wide::TY}, {Square::TX, Square::TY}, {Small::TX, Small::TY}};
+  for (const auto &t : tiles) {
+    b.tx = t[0];
+    b.ty = t[1];
+    if (b.small() && b.precision != TXA_FP32) continue;
     for (int sl : slabs) {
       TXA_HIP(hipStreamSynchronize(s));
       batch_build_items(b, sl);
       for (int g : grids) {
+        if (b.small() && g > ncu) break;
         b.grid = g;
         batch_enqueue(b, s, err);   // warm-up
         TXA_HIP(hipEventRecord(e0, s));
@@ -1391,7 +1404,7 @@ double batch_tune(Batch &b, const txa_assembly_args *args, hipStream_t s, int re
         TXA_HIP(hipEventSynchronize(e1));
         float ms = 0.f;
         TXA_HIP(hipEventElapsedTime(&ms, e0, e1));
-        if (ms / reps < best) { best = ms / reps; best_slab = sl; best_grid = g; best_tx = tx; }
+        if (ms / reps < best) { best = ms / reps; best_slab = sl; best_grid = g; best_tx = t[0]; best_ty = t[1]; }
       }
     }
   }
@@ -1399,6 +1412,7 @@ double batch_tune(Batch &b, const txa_assembly_args *args, hipStream_t s, int re
   (void)hipEventDestroy(e1);
   TXA_HIP(hipStreamSynchronize(s));
   b.tx = best_tx;
+  b.ty = best_ty;
   batch_build_items(b, best_slab);
   b.grid = best_grid;
   TXA_HIP(hipEventRecord(b.done, s));
@@ -1406,13 +1420,17 @@ double batch_tune(Batch &b, const txa_assembly_args *args, hipStream_t s, int re
   return best;
 }
 
-// The work shape set by hand (what the autotuner would otherwise pick): tile width,
-// slab height and persistent grid.  No launch of the batch may be in flight.
-void batch_shape(Batch &b, int tile_x, int slab, int grid) {
-  TXA_REQUIRE(tile_x == 16 || tile_x == 32, TXA_ERR_INVALID, "tile width must be 16 or 32");
+// The work shape set by hand (what the autotuner would otherwise pick): tile (width, with the height in
+// the bits above 16, 0: 256 / width), slab height and persistent grid.  No launch of the batch may be in flight.
+void batch_shape(Batch &b, int tile, int slab, int grid) {
+  const int tx = tile & 0xffff, ty = tile >> 16;
+  const bool small = tx == Small::TX && ty == Small::TY && b.precision == TXA_FP32;
+  TXA_REQUIRE(small || ((tx == Square::TX || tx == Wide::TX) && (ty == 0 || ty == 256 / tx)), TXA_ERR_INVALID,
+              "the tile must be 32 x 8, 16 x 16 or, in FP32, 16 x 8");
   TXA_REQUIRE(slab >= 0 && grid >= 1, TXA_ERR_INVALID, "slab must be >= 0 (0: whole column) and grid >= 1");
   if (b.launched) TXA_HIP(hipEventSynchronize(b.done));
-  b.tx = tile_x;
+  b.tx = tx;
+  b.ty = ty == 0 ? 256 / tx : ty;
   b.grid = grid;
   batch_build_items(b, slab);
 }
@@ -1422,7 +1440,7 @@ void batch_info(const Batch &b, int64_t *out) {
   out[1] = static_cast<int64_t>(b.items_h.size());
   out[2] = b.slab;
   out[3] = b.grid;
-  out[4] = b.tx;
+  out[4] = b.small() ? b.tx | b.ty << 16 : b.tx;
   out[5] = b.mixed ? 1 : 2;
 }
 
