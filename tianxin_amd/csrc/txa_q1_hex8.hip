@@ -1023,7 +1023,7 @@ Q1Plan q1_plan(const Mesh &m, int ncu) {
     const int64_t tiles = static_cast<int64_t>(tiles_x(m, Small::TX)) * tiles_y(m, Small::TY);
     int zc = layers, last = 0;
     *cost = 1e300;
-    for (int n = 1; n <= layers; ++n) {
+    for (int n = 1; n <= std::min(layers, 65535); ++n) {   // slabs run along the grid's z: 65,536 at most
       const int z = (layers + n - 1) / n;
       if (z == last) continue;
       last = z;
