@@ -81,10 +81,11 @@ def cpu_baseline(n=128, reps=10, n1=48, reps1=10):
 
 
 COPY_BYTES = 1 << 30
-# the unit cube's cells are parallelepipeds: the one-metric hex8 kind (17); jittered cells run kind 1
-FP32_KERNEL = "k_q1_hex8_diffusion<17, float, false, false>"   # FP32 integration, steady
-FP64_KERNEL = "k_q1_hex8_diffusion<17, double, false, true>"   # FP64, steady, beta = 1
-FP32_KERNEL_GENERAL = "k_q1_hex8_diffusion<1, float, false, false>"
+# the unit cube's cells are parallelepipeds: the one-metric hex8 kind (17) on 16 x 8 tiles; jittered cells
+# run kind 1, at 256^3 on 32 x 8 tiles
+FP32_KERNEL = "k_q1_hex8_diffusion<Tile<16, 128>, 17, float, false, false>"   # FP32 integration, steady
+FP64_KERNEL = "k_q1_hex8_diffusion<Tile<16, 128>, 17, double, false, true>"   # FP64, steady, beta = 1
+FP32_KERNEL_GENERAL = "k_q1_hex8_diffusion<Tile<32, 256>, 1, float, false, false>"
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "q1_hex8_diffusion_fp32_256_traffic.json")
 
 
@@ -105,15 +106,16 @@ def _rows(d, suffix):
     return rows
 
 
+def _short(name):
+    """A demangled kernel name without its namespaces, return type and parameters."""
+    return name.replace("(anonymous namespace)::", "").replace("txa::", "").replace("void ", "").split("(")[0].strip()
+
+
 def _match(name, kernel):
-    """Demangled-name match of a kernel instance: 'k_q1_hex8_ring<1, float, false>'."""
-    base, targs = kernel.split("<", 1)
-    targs = [t.strip() for t in targs.rstrip(">").split(",")]
-    if base not in name:
-        return False
-    inside = name.split(base, 1)[1]
-    return all(t in inside.split("(")[0] for t in targs) and inside.split("(")[0].replace(" ", "").startswith(
-        "<" + ",".join(targs))
+    """Whether a demangled name is the kernel instance 'k_name<template arguments>', or, without
+    arguments, any instance of it."""
+    short = _short(name)
+    return short.replace(" ", "") == kernel.replace(" ", "") or ("<" not in kernel and short.split("<")[0] == kernel)
 
 
 def _counter_per_dispatch(d, counter, pred, last=None):
@@ -672,11 +674,12 @@ def bench_serve(args):
     return line
 
 
-Q2_KERNELS = {"split_bf16": "k_elastic<27, 27, 256, 2>", "fp32": "k_elastic<27, 27, 256, 1>",
-              "fp64": "k_elastic<27, 27, 256, 0>"}
-# second phase (node-centric gather) of each form: FP32 element blocks, FP64 in the FP64 form
+# first and second kernel of each form: element kernel and node gather; in FP64 the points of each cell
+# and the line kernel
+Q2_KERNELS = {"split_bf16": "k_elastic<27, 27, 256, 2>", "fp32": "k_elastic<27, 27, 256, 1>", "fp64": "k_points27"}
 Q2_GATHER = {"split_bf16": "k_elastic_gather<27, float>", "fp32": "k_elastic_gather<27, float>",
-             "fp64": "k_elastic_gather<27, double>"}
+             "fp64": "k_elastic27_nodes<false>"}
+Q2_COUNTED = dict(Q2_KERNELS, fp64=Q2_GATHER["fp64"])   # the kernel with the form's matrix products
 
 
 def bench_upload(args):
@@ -912,17 +915,19 @@ def summarize_q2(stats_dir, pmc_dir):
              "python3 bench.py --workload q2 --steps 3 --warmup 1",
              f"    rocprofv3 --pmc {pmc_list} --output-format csv -d <out>/pmc_q2 -- "
              "python3 bench.py --workload q2 --steps 1 --warmup 0", "",
-             "Each form is two kernels: the element kernel (geometry, Gram matrix, element block and",
-             "residual to a workspace) and the node-centric gather (sums the blocks around each node into",
-             "its CRS rows, writes each row once), each launched once per z slab (8 slabs of 8 element",
+             "The split-BF16 and FP32 forms are two kernels: the element kernel (geometry, Gram matrix, element",
+             "block and residual to a workspace) and the node-centric gather (sums the blocks around each node",
+             "into its CRS rows, writes each row once), each launched once per z slab (8 slabs of 8 element",
              "layers): the elements on one stream, each slab's node planes gathered on another once its",
-             "elements are done, so slab k+1's element kernel runs beside slab k's gather.  From the",
-             "kernel trace, per step: the span from the first element dispatch's start to the last",
-             "gather dispatch's end, and the summed durations of each kernel's dispatches (their sum",
+             "elements are done, so slab k+1's element kernel runs beside slab k's gather.  The FP64 form is",
+             "`k_points27` (each cell's quadrature points) and `k_elastic27_nodes` (a wave per line of nodes, no",
+             "element blocks), one after the other.  From the",
+             "kernel trace, per step: the span from the first kernel's first start to the second's",
+             "last end, and the summed durations of each kernel's dispatches (their sum",
              "exceeds the span by the overlap).  Rates are over the span; the HBM fraction counts the",
              "compulsory bytes (CRS values and f written once, x read: "
              f"{Q2_BYTES_PER_ELEM / 1e3:.1f} KB per element) against 8 TB/s.", "",
-             "| form | step span ms | element kernel ms (summed) | gather ms (summed) | overlap ms | elements/s | "
+             "| form | step span ms | first kernel ms (summed) | second kernel ms (summed) | overlap ms | elements/s | "
              "dense TFLOP/s | HBM fraction |",
              "|---|---:|---:|---:|---:|---:|---:|---:|"]
     trace = sorted(_rows(stats_dir, "kernel_trace.csv"), key=lambda r: int(r["Start_Timestamp"]))
@@ -960,16 +965,16 @@ def summarize_q2(stats_dir, pmc_dir):
                      f"{Q2_BYTES_PER_ELEM * nel / (ms / 1e3) / HBM_PEAK:.3f} |")
     lines += ["", "Other kernels of the run (setup included):", "", "| kernel | calls | average ms |", "|---|---:|---:|"]
     for r in sorted(stats, key=lambda r: -float(r["TotalDurationNs"]))[:8]:
-        if "k_elastic" not in r["Name"]:
+        if "k_elastic" not in r["Name"] and "k_points27" not in r["Name"]:
             lines.append(f"| `{r['Name'][:80]}` | {r['Calls']} | {float(r['AverageNs']) / 1e6:.3f} |")
     per = {}
     for r in _rows(pmc_dir, "counter_collection.csv"):
-        for name, k in Q2_KERNELS.items():
+        for name, k in Q2_COUNTED.items():
             if _match(r.get("Kernel_Name", ""), k):
                 d = per.setdefault(name, {})
                 key = (int(r["Dispatch_Id"]), r["Counter_Name"])
                 d[key] = d.get(key, 0.0) + float(r["Counter_Value"])
-    lines += ["", "## Element-kernel counters (one dispatch each)", "",
+    lines += ["", "## Counters (element kernels; FP64: the line kernel)", "",
               "| form | MFMA busy (of all SIMD cycles) | VALU wave-instructions / element | "
               "MFMA bf16 MOPs / element | MFMA f64 MOPs / element | LDS wave-instructions / element |",
               "|---|---:|---:|---:|---:|---:|"]
@@ -982,14 +987,17 @@ def summarize_q2(stats_dir, pmc_dir):
             vals = list(tot.get(c, {}).values())
             return sum(vals) / len(vals) if vals else float("nan")
         simds = 256 * 4
-        util = avg("SQ_VALU_MFMA_BUSY_CYCLES") / (avg("GRBM_GUI_ACTIVE") * simds) if avg("GRBM_GUI_ACTIVE") else 0
-        lines.append(f"| {name} | {100 * util:.1f}% | {avg('SQ_INSTS_VALU') / nel:.0f} | "
-                     f"{avg('SQ_INSTS_VALU_MFMA_MOPS_BF16') / nel:.3g} | {avg('SQ_INSTS_VALU_MFMA_MOPS_F64') / nel:.3g} | "
-                     f"{avg('SQ_INSTS_LDS') / nel:.0f} |")
+        # GRBM_GUI_ACTIVE is summed over the 8 XCDs
+        util = avg("SQ_VALU_MFMA_BUSY_CYCLES") / (avg("GRBM_GUI_ACTIVE") / 8 * simds) if avg("GRBM_GUI_ACTIVE") else 0
+        nd = nel if name == "fp64" else nel / 8   # elements per dispatch: the element kernels run in 8 slabs
+        lines.append(f"| {name} | {100 * util:.1f}% | {avg('SQ_INSTS_VALU') / nd:.0f} | "
+                     f"{avg('SQ_INSTS_VALU_MFMA_MOPS_BF16') / nd:.3g} | {avg('SQ_INSTS_VALU_MFMA_MOPS_F64') / nd:.3g} | "
+                     f"{avg('SQ_INSTS_LDS') / nd:.0f} |")
     lines += ["", "The split-BF16 form runs six v_mfma_f32_16x16x32_bf16 products per 16x16 tile (21",
-              "upper-triangle tiles, one K = 32 step over the 27 points), the FP64 form one",
-              "v_mfma_f64_16x16x4f64 and the FP32 form one v_mfma_f32_16x16x4f32 per tile and k-step (21",
-              "tiles, 7 k-steps; the FP32 MOPs are counted by neither column).  The element kernels run one",
+              "upper-triangle tiles, one K = 32 step over the 27 points), the FP32 form one",
+              "v_mfma_f32_16x16x4f32 per tile and k-step (21 tiles, 7 k-steps; the FP32 MOPs are counted by",
+              "neither column).  The FP64 line kernel forms each cell's blocks once per line that the cell",
+              "touches (nine), six v_mfma_f64_16x16x4f64 per k-step.  The element kernels run one",
               "element per workgroup through barrier-separated",
               "phases (loads, geometry, gradients, Gram matrix, pair blocks, block store), so per-element",
               "latency, not the MFMA rate, sets their time; the gather moves the workspace blocks in and",
@@ -1033,22 +1041,25 @@ def summarize_batch(stats_dir, bench_json):
                     "k_dirichlet_batch" in r["Kernel_Name"]})
     for n in names:
         d = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in trace if r["Kernel_Name"] == n]
-        short = n.replace("txa::(anonymous namespace)::", "").replace("void ", "").split("(")[0]
+        short = _short(n)
         lines.append(f"| `{short}` | {len(d)} | {np.mean(d):.1f} | {np.min(d):.1f} | {np.max(d):.1f} |")
     # the timed FP32 graph replays: the last `steps` dispatches of the chosen shape's float kernels
-    tx = int(f32["tile"].split("x")[0])
+    tx, ty = (int(v) for v in f32["tile"].split("x"))
     steps = BATCH_PROF_STEPS
     lines += ["", f"Timed FP32 steps (the last {steps} dispatches of the {f32['tile']} float kernels):", ""]
     for n in names:
-        if f"<{tx}, " not in n or "float" not in n:
+        if f"<Tile<{tx}, {tx * ty}>, " not in _short(n) or "float" not in n:
             continue
         rs = sorted((r for r in trace if r["Kernel_Name"] == n), key=lambda r: int(r["Start_Timestamp"]))[-steps:]
         d = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in rs]
-        short = n.replace("txa::(anonymous namespace)::", "").replace("void ", "").split("(")[0]
+        short = _short(n)
         lines.append(f"- `{short}`: mean {np.mean(d):.1f} us over {len(d)} dispatches")
     out = os.path.join(ROOT, "profiles", "batch_512_kernel_stats.md")
     open(out, "w").write("\n".join(lines) + "\n")
     print(out)
+
+
+ELASTIC_KERNELS = ("k_elastic8_affine", "k_elastic8_general", "k_elastic8_upload")
 
 
 def summarize_elastic(stats_dir, pmc_dir, bench_json):
@@ -1067,11 +1078,9 @@ def summarize_elastic(stats_dir, pmc_dir, bench_json):
              "python3 bench.py --workload elastic --steps 2 --warmup 0", "",
              "Workload: " + line["config"]["workload"] + ", E lognormal (sigma 0.3) per cell, Rayleigh damping,",
              "Newmark seeds (alpha 2000, gamma2 4e6), u = 0 on x = 0; a step is one assembly with the",
-             "Dirichlet rows.  Parallelepiped cells (the unit cube) take the node-centric kernel",
-             "`k_elastic8_affine` (closed-form blocks, no workspace); jittered cells take the element",
-             "kernel `k_elastic<8, 8, 64, 0>` and the gather `k_elastic_gather<8, double>` in 8 z slabs on two",
-             "streams (8 dispatches of each per step, the gather of slab k beside the element kernel of slab",
-             "k+1); the uploaded mesh runs the element kernel once and `k_elastic_gather_u` once per step.", "",
+             "Dirichlet rows.  Each call is one node kernel without a workspace: `k_elastic8_affine` for",
+             "parallelepiped cells (the unit cube; closed-form blocks), `k_elastic8_general` for the jittered",
+             "brick, `k_elastic8_upload` for the uploaded mesh.", "",
              "| cells | ms per step (HIP events) | p50 / p99 ms | elements/s | HBM fraction (compulsory bytes) |",
              "|---|---:|---:|---:|---:|"]
     for name, c in line["cells"].items():
@@ -1084,37 +1093,34 @@ def summarize_elastic(stats_dir, pmc_dir, bench_json):
                      f"{c['ms_per_step']:.3f} | | {c['elements_per_s']:.3g} | |")
     up = line["cells"].get("jittered_cells_uploaded", {}).get("brick_order", {}).get("vs_brick_normwise")
     if up:
-        lines += ["", "The uploaded mesh (element kernel, then `k_elastic_gather_u`: each node's element instances",
-                  "from its list, slot maps per instance) in brick order against the brick's lattice gather: "
-                  f"R {up['R']:.1e}, J {up['J']:.1e} normwise."]
+        lines += ["", "The uploaded mesh (each node's element instances from its list, slot maps per instance) in brick",
+                  f"order against the brick: R {up['R']:.1e}, J {up['J']:.1e} normwise."]
     lines += ["", "Per-dispatch durations from the kernel trace (us), all dispatches of the run:", "",
               "| kernel | calls | mean | min | max |", "|---|---:|---:|---:|---:|"]
-    for k in ("k_elastic8_affine", "k_elastic<8, 8, 64, 0>", "k_elastic_gather<8, double>",
-              "k_elastic_gather_u<8, double>", "k_dirichlet"):
-        d = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in trace
-             if (k in r["Kernel_Name"] if "<" not in k else _match(r["Kernel_Name"], k))]
+    for k in ELASTIC_KERNELS + ("k_dirichlet",):
+        d = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3 for r in trace if _match(r["Kernel_Name"], k)]
         if d:
             lines.append(f"| `{k}` | {len(d)} | {np.mean(d):.1f} | {np.min(d):.1f} | {np.max(d):.1f} |")
-    tot = {}
-    for r in _rows(pmc_dir, "counter_collection.csv"):
-        if "k_elastic8_affine" in r.get("Kernel_Name", ""):
-            tot.setdefault(r["Counter_Name"], {}).setdefault(r["Dispatch_Id"], 0.0)
-            tot[r["Counter_Name"]][r["Dispatch_Id"]] += float(r["Counter_Value"])
-    if tot:
+    rows = [r for r in _rows(pmc_dir, "counter_collection.csv")]
+    nodes = 129 ** 3
+    lines += ["", "## Counters (per dispatch, per lattice node)", "",
+              "| kernel | VALU wave-instructions | LDS | SALU | vector memory reads | waves per dispatch | "
+              "VALU busy (of SIMD cycles) |", "|---|---:|---:|---:|---:|---:|---:|"]
+    for k in ELASTIC_KERNELS:
+        tot = {}
+        for r in rows:
+            if _match(r.get("Kernel_Name", ""), k):
+                tot.setdefault(r["Counter_Name"], {}).setdefault(r["Dispatch_Id"], 0.0)
+                tot[r["Counter_Name"]][r["Dispatch_Id"]] += float(r["Counter_Value"])
+        if not tot:
+            continue
         avg = {c: sum(v.values()) / len(v) for c, v in tot.items()}
-        nodes = 129 ** 3
-        lines += ["", "## `k_elastic8_affine` counters (per dispatch, per lattice node)", "",
-                  f"- VALU wave-instructions per node: {avg.get('SQ_INSTS_VALU', 0) / nodes:.0f}; LDS: "
-                  f"{avg.get('SQ_INSTS_LDS', 0) / nodes:.0f}; SALU: {avg.get('SQ_INSTS_SALU', 0) / nodes:.0f}; "
-                  f"vector memory reads: {avg.get('SQ_INSTS_VMEM_RD', 0) / nodes:.0f}",
-                  f"- waves per dispatch: {avg.get('SQ_WAVES', 0):.0f}; GRBM_GUI_ACTIVE (summed over the 8 XCDs): "
-                  f"{avg.get('GRBM_GUI_ACTIVE', 0):.3g}",
-                  "- one wave per node: 8 cells x 8 vertices on the 64 lanes, a 3x3 block per lane from the",
-                  "  cell's scaled cofactors and |det J| (a per-mesh table, `k_cell_geom`): Chat S Chat^T, the",
-                  "  Newmark/Rayleigh combination, eight cell-ordered LDS adds, rows stored non-temporally.",
-                  "  Timing probes (work skipped) put the LDS adds and the state loads' dependence on the",
-                  "  LIDs at 1% each and the row stores at about 0.3 ms: the VALU work and its dependences",
-                  "  (four waves per SIMD at 125 VGPRs) set the rest."]
+        lines.append(f"| `{k}` | {avg['SQ_INSTS_VALU'] / nodes:.0f} | {avg['SQ_INSTS_LDS'] / nodes:.0f} | "
+                     f"{avg['SQ_INSTS_SALU'] / nodes:.0f} | {avg['SQ_INSTS_VMEM_RD'] / nodes:.0f} | {avg['SQ_WAVES']:.0f} | "
+                     f"{4 * avg['SQ_INSTS_VALU'] / (1024 * avg['GRBM_GUI_ACTIVE'] / 8):.2f} |")
+    lines += ["", "VALU busy = 4 x SQ_INSTS_VALU / (1024 SIMDs x GRBM_GUI_ACTIVE / 8).  The affine kernel runs a wave",
+              "per line of four nodes along x, the general one 16 nodes per workgroup over one table of their 50",
+              "cells' points, the upload one two nodes per wave with the points of each node's own cells."]
     out = os.path.join(ROOT, "profiles", "elastic_hex8_128_kernel_stats.md")
     open(out, "w").write("\n".join(lines) + "\n")
     print(out)
@@ -1497,7 +1503,9 @@ def main():
     achieved = BYTES_PER_ELEM * nel / (kt32 / 1e3) / 1e9
     traffic = None
     if n == 256 and os.path.exists(TRAFFIC_FILE):
-        traffic = json.load(open(TRAFFIC_FILE)).get("bytes_per_launch")
+        counted = json.load(open(TRAFFIC_FILE))
+        if counted.get("kernel") == FP32_KERNEL:   # counters of another kernel say nothing about this one
+            traffic = counted.get("bytes_per_launch")
     out = {
         "metric": "elements/s (residual+Jacobian) vs plain FP64 at stated error; p50/p99 latency",
         "value": value, "unit": "elements/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
