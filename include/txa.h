@@ -312,8 +312,10 @@ int txa_model_destroy(txa_ctx ctx, int model_id);
  * element blocks of the two-phase elasticity kernels, the element matrices of the
  * multi-block row gather, the curve-ordered state of a scattered node-patch mesh)
  * comes from one static device array of 128 MiB per
- * device instead of the context's pool; an assembly that needs more is refused with
- * TXA_ERR_NOMEM before anything is launched.  Results equal txa_assemble's.  Every
+ * device instead of the context's pool; an assembly sized above that is refused with
+ * TXA_ERR_NOMEM before anything is launched (the size counts the element blocks of every
+ * elasticity call but hex8 bricks of parallelepiped cells, also where FP64 kernels do
+ * without them: the accepted sizes do not move with the kernels).  Results equal txa_assemble's.  Every
  * call on one device shares that array: calls whose work overlaps on one GPU (other
  * streams, other contexts, other threads) race and must be ordered by the caller. */
 int txa_assemble_noalloc(txa_ctx ctx, int mesh_id, const txa_assembly_args *args, void *stream);

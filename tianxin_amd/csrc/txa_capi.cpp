@@ -329,9 +329,9 @@ int txa_assemble_noalloc(txa_ctx ctx, int mesh_id, const txa_assembly_args *args
     const size_t wsb = txa::assemble_workspace_bytes(m, args->physics, args->precision, args->f != nullptr,
                                                      args->vals != nullptr, args->accumulate != 0, true);
     TXA_REQUIRE(wsb <= kScratchBytes, TXA_ERR_NOMEM,
-                "txa_assemble_noalloc: this assembly needs " + std::to_string(wsb) +
-                    " bytes of workspace; the static workspace holds " + std::to_string(kScratchBytes) +
-                    " (use txa_assemble)");
+                "txa_assemble_noalloc: this assembly is sized at " + std::to_string(wsb) +
+                    " bytes of workspace (element blocks counted where the kernel does without them, too); the static"
+                    " workspace holds " + std::to_string(kScratchBytes) + " (use txa_assemble)");
     TXA_REQUIRE(ctx->scratch != nullptr, TXA_ERR_LOGIC, "static workspace not set up");
     txa::assemble(m, *args, static_cast<hipStream_t>(stream), wsb ? ctx->scratch : nullptr, ctx->err.p);
   });
