@@ -1167,7 +1167,9 @@ __global__ __launch_bounds__(256, 3) void k_elastic8_affine(Elastic8Params p) {
   const double cK = TR ? p.beta + p.alpha * p.rb : p.beta;
   const double cM = TR ? p.alpha * p.ra + (tra ? p.gamma2 : 0.0) : 0.0;
   double vu[3], vm[3], En;
-  int32_t Ln;
+  // LID of this lane's node; its cell (one outside the mesh: the nearest, which has this node and every
+  // vertex that the two share, so a degenerate cell reaches the rows of its own vertices only)
+  int32_t Ln, Cn;
   auto load_tile = [&](int tile) {
     const int I0 = tile % gx * kN8, J0 = tile / gx % gy, K = tile / (gx * gy);
     const int t = min(lane, NV - 1);
@@ -1187,7 +1189,8 @@ __global__ __launch_bounds__(256, 3) void k_elastic8_affine(Elastic8Params p) {
     Ln = p.point_lid[3 * (min(I0 + n, p.nx) + sx * J0 + sxy * K)];
     const int cx = min(max(I0 + n - 1 + q.ox, 0), p.nx - 1), cy = min(max(J0 - 1 + q.oy, 0), p.ny - 1),
               cz = min(max(K - 1 + q.oz, 0), p.nz - 1);
-    En = p.coef[cx + p.nx * (cy + p.ny * cz)];
+    Cn = cx + p.nx * (cy + p.ny * cz);
+    En = p.coef[Cn];
   };
   const int stride = static_cast<int>(gridDim.x) * 4;
   int tile = static_cast<int>(blockIdx.x) * 4 + w;
@@ -1211,10 +1214,7 @@ __global__ __launch_bounds__(256, 3) void k_elastic8_affine(Elastic8Params p) {
     const bool cell_ok = node_ok && cx >= 0 && cx < p.nx && cy >= 0 && cy < p.ny && cz >= 0 && cz < p.nz;
     const double E = cell_ok ? En : 0.0;
     double2 G[5];
-    // an absent cell takes the geometry of the nearest one, which has this node and every vertex that the
-    // two share: a degenerate cell reaches the rows of its own vertices only
-    const int gx_ = min(max(cx, 0), p.nx - 1), gy_ = min(max(cy, 0), p.ny - 1), gz_ = min(max(cz, 0), p.nz - 1);
-    const double2 *gp = reinterpret_cast<const double2 *>(p.geom + 10 * static_cast<int64_t>(gx_ + p.nx * (gy_ + p.ny * gz_)));
+    const double2 *gp = reinterpret_cast<const double2 *>(p.geom + 10 * static_cast<int64_t>(Cn));
 #pragma unroll
     for (int t = 0; t < 5; ++t) G[t] = gp[t];
     const int64_t base = p.rowptr[L0];
