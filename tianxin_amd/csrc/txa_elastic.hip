@@ -1015,19 +1015,15 @@ __global__ void k_node_perm(int64_t px, int64_t py, int64_t pz, int R, int nf, i
 }
 
 // Affine HEX8 bricks (every cell a parallelepiped), three fields: node-centric assembly with
-// no workspace.  One wave per lattice node.  Lane (c, b) = (cell c of the eight around the
-// node, vertex b of that cell, binary order) forms the 3x3 block of the node's vertex a and b in
-// closed form: with J = dx/dxi constant over the cell and C its cofactor matrix,
+// no workspace.  The 3x3 block of a node's vertex a and another vertex b of a cell has a closed
+// form: with J = dx/dxi constant over the cell and C its cofactor matrix,
 //   T_ab = |det J| J^-T S_ab J^-1 = C S_ab C^T / |det J|,
 //   S_ab[m][n] = sum_q dN_a/dxi_m dN_b/dxi_n   (2x2x2 Gauss)
 //              = s_a^m s_b^n f_d / 4 (m != n, d the third axis),  s_a^m s_b^m f_d1 f_d2 / 2 (m = n),
 // with s the vertex's sign along an axis and f = 2/3 where a and b share it, 1/3 otherwise;
-// the mass entry rho |det J| f_x f_y f_z, the source load src |det J| per vertex.  The rows are
-// summed in LDS in eight steps, one per cell in a fixed order: in step c the cell's eight lanes
-// (eight distinct neighbours) add their blocks at the neighbours' positions (from nperm); one
-// wave's LDS operations execute in order, so every entry is summed in cell order and the result
-// is bitwise reproducible.  The wave then writes the node's three rows once, coalesced.  The
-// general (per-point) form is the element kernel plus the gather.
+// the mass entry rho |det J| f_x f_y f_z, the source load src |det J| per vertex.  Blocks of
+// cells that share a vertex are summed in a fixed order (bitwise reproducible), each node's three
+// rows written once (k_elastic8_affine).
 struct Elastic8Params {
   int nx, ny, nz;
   int64_t npoints;
@@ -1137,14 +1133,15 @@ __device__ __forceinline__ void store_line(const double *rows, double *vals, int
   }
 }
 
-// One wave per line of four nodes along x, 16 lanes per node; each lane forms the blocks of its cell's four vertices on one z side one after another.  With the
-// cell's cofactor columns signed by the node's corner (c_m s_a^m), T_ab = sum_mn c_m F_mn sigma_n c_n^T
-// where sigma_n = +1 / -1 and f_n = 2/3 / 1/3 as a and b agree or not along n, F_mm = f_d1 f_d2 / 2,
-// F_mn = f_d / 4 (d the third axis): x and y known per block, z per lane.  The state of the 6 x 3 x 3
-// vertices is staged in LDS, the next line's loaded before this line's row stores (one counter tracks
-// a wave's loads and stores); the waves of a workgroup share nothing.
+// One wave per line of four nodes along x, 16 lanes per node; each lane forms the blocks of its cell's
+// four vertices on one z side one after another.  With the cell's cofactor columns signed by the node's
+// corner (c_m s_a^m), T_ab = sum_mn c_m F_mn sigma_n c_n^T where sigma_n = +1 / -1 and f_n = 2/3 / 1/3 as a
+// and b agree or not along n, F_mm = f_d1 f_d2 / 2, F_mn = f_d / 4 (d the third axis): x and y known per
+// block, z per lane.  The state of the 6 x 3 x 3 vertices is staged in LDS, the next line's loaded before
+// this line's row stores (one counter tracks a wave's loads and stores); the waves of a workgroup share
+// nothing.
 //
-// Bound by VALU issue (297 instructions per node, 73% busy at three waves per SIMD) and the row
+// Bound by VALU issue (296 instructions per node, 67% busy at three waves per SIMD) and the row
 // stores.  Transient FP64, against one wave per node with 64 lanes of one block each, eight ordered
 // LDS adds per entry and the state loaded once per lane (390 instructions per node): 128^3 2.56 ->
 // 1.71 ms, 115^3 1.82 -> 1.22 ms, 64^3 319 -> 229 us; the same tiles staged per workgroup behind two
@@ -1466,8 +1463,8 @@ __device__ __forceinline__ void row_blocks(const double *tab, int bb, int fa, do
 // z in that order, one lane then writes each neighbour's block into the row buffer (which lies over
 // the point table) and the wave stores the rows, its four nodes as one range where their LIDs follow
 // each other.  Every sum has a fixed order: results are bitwise reproducible.
-// Bound by VALU issue (about 520 instructions per node, 65% busy at two workgroups per CU, 208
-// VGPRs; held to 168 for three it spills and takes 18% longer).  Transient FP64, against the element
+// Bound by VALU issue (about 515 instructions per node, 63% busy at two workgroups per CU, 208
+// VGPRs; held to 168 for three it spills and takes 18% longer) and waits (32% of wave time).  Transient FP64, against the element
 // kernel with its 4.6 KB of blocks per element and the gather: 128^3 8.23 -> 2.84 ms, 96^3 3.61 ->
 // 1.21 ms, 18^3 238 -> 28 us.
 struct Elastic8GParams {
@@ -1655,11 +1652,12 @@ __global__ __launch_bounds__(256, 2) void k_elastic8_general(Elastic8GParams gp)
 
 // The same row blocks on an uploaded hex8 mesh (one block): one wave per two nodes (LIDs 3 n, 3 n + 1,
 // 3 n + 2), 32 lanes per node: lane (element instance c of eight at a time, corner y and z) forms the
-// blocks of the two vertices along x.  Bound by latency at two waves per SIMD (245 VGPRs, 16 KB of LDS
-// per wave) and VALU issue (about 800 instructions per node: no two nodes share a point table).
-// Transient FP64, shuffled 64x61x67: 1.19 -> 0.63 ms (element kernel and gather before).  Instances come from the node's list (ascending), the row
-// positions from their slot maps; the blocks are added into the node's rows in LDS instance by
-// instance, so the sums have a fixed order, and the rows are stored once.
+// blocks of the two vertices along x.  Bound by LDS (70% busy: points and row adds) and VALU issue (about
+// 657 instructions per node, 47% busy: no two nodes share a point table) at two waves per SIMD (245 VGPRs,
+// 16 KB of LDS per wave).  Transient FP64, shuffled 64x61x67: 1.19 -> 0.64 ms (element kernel and gather
+// before).  Instances come from the node's list (ascending), the row positions from their slot maps; the
+// blocks are added into the node's rows in LDS instance by instance, so the sums have a fixed order, and
+// the rows are stored once.
 struct Elastic8UParams {
   Elastic8Params p;
   const double *X, *Y, *Z;
@@ -1860,8 +1858,8 @@ __global__ __launch_bounds__(64, 2) void k_elastic8_upload(Elastic8UParams gp) {
 // line), and rows are stored once in CRS order when their last cell is done.
 //
 // Bound by issue: an FP64 product takes its SIMD's 64 cycles whole (a wave's VALU work, and the other
-// waves', wait for it: measured), 0.9 M of 2.6 M cycles per SIMD at 33^3 (46% of its rows and columns are
-// used), and 218 k VALU instructions 0.87 M more, at seven waves per CU (23 KB of LDS each).  FP64 33^3,
+// waves', wait for it: measured), 0.90 M of 2.71 M cycles per SIMD at 33^3 (46% of its rows and columns are
+// used), and 238 k VALU instructions 0.95 M more, at seven waves per CU (23 KB of LDS each).  FP64 33^3,
 // against the element kernel with its 55 KB of blocks per element and the gather: steady 1.79 -> 1.17 ms,
 // transient 2.16 -> 1.72 ms (with the mass matrix on the products too, 2.29 ms: it spilled); 12^3 steady
 // 225 -> 125 us, transient 263 -> 150 us, 4^3 steady 124 -> 48 us.
@@ -2607,7 +2605,8 @@ void launch_elastic(Mesh &m, const txa_assembly_args &a, hipStream_t s, void *ws
   // on that stream: no streams or events are created inside a capture.
   // A slab below some 24,000 elements costs more in launches, events and emptied CUs than the overlap
   // gives (hex27 split, one slab against eight: 8^3 48 and 174 us, 20^3 273 and 366, 36^3 1374 and 1459;
-  // four against one and eight: 46^3 2801, 2848 and 2865 us; eight against four: 64^3 7.40 and 7.48 ms).
+  // four against one and eight: 46^3 2801, 2848 and 2865 us; eight against four: 64^3 7.40 and 7.48 ms;
+  // hex8 FP32 on general cells, against eight: 32^3 in one 121 and 250 us, 48^3 in four 397 and 443).
   const int nslab = std::min({kSlabs, m.nz, static_cast<int>(std::min<int64_t>(m.nelem / 24000, kSlabs))});
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   TXA_HIP(hipStreamIsCapturing(s, &cs));
