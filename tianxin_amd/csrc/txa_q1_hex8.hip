@@ -95,10 +95,11 @@ __device__ __forceinline__ double dot3(double a0, double b0, double a1, double b
   return __builtin_fma(a2, b2, __builtin_fma(a1, b1, a0 * b0));
 }
 
-// x / 6, correctly rounded: the product with 1/6 and its remainder (three operations, a division eleven)
+// x / 6, correctly rounded: the product with 1/6 and its remainder, Inf kept (four operations, a division
+// eleven)
 __device__ __forceinline__ double sixth(double x) {
   const double q = x * (1.0 / 6.0);
-  return __builtin_fma(__builtin_fma(-6.0, q, x), 1.0 / 6.0, q);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-6.0, q, x), 1.0 / 6.0, q), 6.0, x);
 }
 
 // The six linear tets of one cell, assembled into the cell's 8x8 matrix (pairs
@@ -1369,10 +1370,10 @@ void batch_assemble(Batch &b, const txa_assembly_args *args, bool use_graph, hip
 
 // Autotuner: times the batch over the tiles, slab heights (the analogue of
 // Panzer's workset size sweep) and persistent grid sizes, keeps the fastest.
-// FP32 tries 16 x 16 beside 16 x 8: it is up to 9% faster where a small batch's
+// FP32 tries 16 x 16 beside 16 x 8: tuned, it is 9% faster where a small batch's
 // items are general hex8 cells (48 meshes of 8-48 cells, transient: 222 us against
-// 243), 16 x 8 up to 18% where there are many (512 meshes: 1.96 ms against 2.2);
-// more 16 x 8 workgroups than the resident ones never won.  out: best ms.
+// 243), 16 x 8 3% where there are many (512 meshes of 8-64 cells: 2.09 ms against
+// 2.15); 16 x 8 runs with its resident workgroups only.  out: best ms.
 double batch_tune(Batch &b, const txa_assembly_args *args, hipStream_t s, int reps, int *err) {
   int dev = 0, ncu = 0;
   TXA_HIP(hipGetDevice(&dev));
